@@ -511,25 +511,30 @@ __global__ void k_l2_final(const double* __restrict__ part, int n, double* __res
     }
 }
 
-// Probe record (ProbeManager::record, probe.cpp:192-216) on the device, one
-// workgroup per probe: the threads form the rounded products w_p * u_c(p),
-// w_p = (Lr[i] Ls[j]) Lt[k], of all the element's nodes at once into LDS; then
-// one thread per component adds them in node order -- the reference's
+// Probe records (ProbeManager::record, probe.cpp:192-216) on the device, one
+// workgroup per probe and step: the threads form the rounded products w_p *
+// u_c(p), w_p = (Lr[i] Ls[j]) Lt[k], of all the element's nodes at once into LDS;
+// then one thread per component adds them in node order -- the reference's
 // operations in its order, in FP64, so the record is bit for bit the host's --
-// into record slot (*slot mod cap).  k_probe_advance moves the slot afterwards
-// (stream order), so every workgroup reads the same slot.
+// into record slot (*slot + step) mod cap.  The sum is one serial chain: its LDS
+// reads are issued eight at a time ahead of the additions.  `stop`
+// (may be null): nonzero where the steps' launch gave up, no record then.
+// k_probe_advance moves the slot afterwards (stream order), so every workgroup
+// reads the same slot.
 template <typename R>
 __global__ void __launch_bounds__(256) k_probe(const R* __restrict__ u, long long cs, long long ns, int nprobes,
                                                const long long* __restrict__ base, const double* __restrict__ lw,
                                                int n1, double* __restrict__ hist, const int* __restrict__ slot,
-                                               int cap) {
+                                               int cap, long long step_stride, const int* __restrict__ stop) {
+    constexpr int kAhead = 8;
     __shared__ double prod[6][kMaxN1 * kMaxN1 * kMaxN1];
-    const int q = blockIdx.x;
+    if (stop && *stop) return;
+    const int q = blockIdx.x, step = blockIdx.y;
     const int np = n1 * n1 * n1;
     const double* Lr = lw + size_t(q) * 3 * n1;
     const double* Ls = Lr + n1;
     const double* Lt = Ls + n1;
-    const R* up = u + base[q] * ns;
+    const R* up = u + step * step_stride + base[q] * ns;
     for (int p = threadIdx.x; p < np; p += blockDim.x) {
         const int i = p % n1, j = (p / n1) % n1, kk = p / (n1 * n1);
         const double w = __dmul_rn(__dmul_rn(Lr[i], Ls[j]), Lt[kk]);
@@ -537,18 +542,28 @@ __global__ void __launch_bounds__(256) k_probe(const R* __restrict__ u, long lon
         for (int c = 0; c < 6; ++c) prod[c][p] = __dmul_rn(w, double(up[p * ns + c * cs]));
     }
     __syncthreads();
-    if (threadIdx.x < 6) {
+    // past the capacity the history is lost either way (the host reports it)
+    const long long at = (long long)*slot + step;
+    if (threadIdx.x < 6 && (gridDim.y == 1 || at < cap)) {
         const int c = threadIdx.x;
         double acc = 0.0;
-        for (int p = 0; p < np; ++p) acc = __dadd_rn(acc, prod[c][p]);  // no contraction: the host sum's roundings
-        hist[(size_t(*slot % cap) * nprobes + q) * 6 + c] = acc;
+        int p = 0;
+        for (; p + kAhead <= np; p += kAhead) {
+            double v[kAhead];
+#pragma unroll
+            for (int x = 0; x < kAhead; ++x) v[x] = prod[c][p + x];
+#pragma unroll
+            for (int x = 0; x < kAhead; ++x) acc = __dadd_rn(acc, v[x]);  // no contraction: the host sum's roundings
+        }
+        for (; p < np; ++p) acc = __dadd_rn(acc, prod[c][p]);
+        hist[(size_t(at % cap) * nprobes + q) * 6 + c] = acc;
     }
 }
 
 // Counts records up to cap + 1 (the overflow the host reports), so a run that
 // never fetches its history cannot wrap the counter.
-__global__ void k_probe_advance(int* p, int cap) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && *p <= cap) *p = *p + 1;
+__global__ void k_probe_advance(int* p, int cap, int n, const int* __restrict__ stop) {
+    if (threadIdx.x == 0 && blockIdx.x == 0 && !(stop && *stop)) *p = min(*p + n, cap + 1);
 }
 
 // Sets *slot = 0 with a kernel (no memset node if a caller captures it).
@@ -799,19 +814,21 @@ hipError_t launch_fill(double* p, long long n, double v, hipStream_t s) {
 
 template <typename R>
 hipError_t launch_probe(const R* u, long long cs, long long ns, int nprobes, const long long* base, const double* lw,
-                        int n1, double* hist, int* slot, int cap, hipStream_t s) {
-    if (nprobes <= 0) return hipSuccess;
+                        int n1, double* hist, int* slot, int cap, hipStream_t s, int nsteps, long long step_stride,
+                        const int* stop) {
+    if (nprobes <= 0 || nsteps <= 0) return hipSuccess;
     if (n1 < 2 || n1 > kMaxN1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_probe<R>, dim3(nprobes), dim3(256), 0, s, u, cs, ns, nprobes, base, lw, n1, hist, slot, cap);
+    hipLaunchKernelGGL(k_probe<R>, dim3(nprobes, nsteps), dim3(256), 0, s, u, cs, ns, nprobes, base, lw, n1, hist, slot, cap,
+                       step_stride, stop);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_probe_advance, dim3(1), dim3(64), 0, s, slot, cap);
+    hipLaunchKernelGGL(k_probe_advance, dim3(1), dim3(64), 0, s, slot, cap, nsteps, stop);
     return hipGetLastError();
 }
 template hipError_t launch_probe<double>(const double*, long long, long long, int, const long long*, const double*, int,
-                                         double*, int*, int, hipStream_t);
+                                         double*, int*, int, hipStream_t, int, long long, const int*);
 template hipError_t launch_probe<float>(const float*, long long, long long, int, const long long*, const double*, int,
-                                        double*, int*, int, hipStream_t);
+                                        double*, int*, int, hipStream_t, int, long long, const int*);
 
 hipError_t launch_zero_int(int* p, hipStream_t s) {
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, s, p);

@@ -75,7 +75,8 @@ hipError_t launch_l2(const R* u, long long cs, long long ns, const double* ref, 
 // then ++*slot (one block; weights lw = Lr, Ls, Lt per probe, 3 n1 doubles).
 template <typename R>
 hipError_t launch_probe(const R* u, long long cs, long long ns, int nprobes, const long long* base, const double* lw,
-                        int n1, double* hist, int* slot, int cap, hipStream_t s);
+                        int n1, double* hist, int* slot, int cap, hipStream_t s, int nsteps = 1,
+                        long long step_stride = 0, const int* stop = nullptr);
 hipError_t launch_zero_int(int* p, hipStream_t s);
 template <typename D, typename S>
 hipError_t launch_convert(D* dst, long long dcs, long long dns, const S* src, long long scs, long long sns, long long n,

@@ -4,6 +4,7 @@
 #include "nw_solver.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -32,12 +33,16 @@ int upload_gll_tables(int device) {
     if (st != NW_OK) return st;
     st = plain_upload_tables(t);
     if (st != NW_OK) return st;
+    st = resident_upload_tables(t);
+    if (st != NW_OK) return st;
     g_tables_done[device] = true;
     return NW_OK;
 }
 
 // LSRK45 coefficients, Carpenter & Kennedy (1994) (dg_solver.cpp:58-69).
 constexpr int kStages = 5;  // LSRK45 stages per step
+constexpr int kResidentSteps = 1024;        // steps of one resident launch, at most
+constexpr long long kSnapBytes = 32 << 20;  // probed elements' fields kept per resident launch
 static const double kRkA[kStages] = {0.0, -567301805773.0 / 1357537059087.0,
                                      -2404267990393.0 / 2016746695238.0, -3550918686646.0 / 2091501179385.0,
                                      -1275806237668.0 / 842570457699.0};
@@ -208,6 +213,9 @@ void Solver::release() {
     drop_graphs();
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
+    if (h_stop) (void)hipHostFree(h_stop);
+    h_stop = nullptr;
+    release_resident();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     ev0 = ev1 = nullptr;
@@ -316,6 +324,7 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
             sg.affine = true;
             seg.push_back(sg);
         }
+        I.seg = static_cast<int>(seg.size()) - 1;
         seg.back().nelt += m.nelt;
         seg.back().affine = seg.back().affine && m.all_affine;
     }
@@ -479,7 +488,9 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
             if ((st = upload_vec(reinterpret_cast<float**>(&d_fw), w32))) return st;
         }
         kernels_per_step = 5 * (static_cast<int>(seg.size()) + (nhalo > 0 ? 2 : 0));
+        if ((st = init_resident(meshes))) return st;
     }
+    for (size_t x = 0; x < seg.size(); ++x) sets[set_of(static_cast<int>(x))].segs.push_back(static_cast<int>(x));
     NW_TRY_HIP(hipStreamSynchronize(stream));
     initialized = true;
     return NW_OK;
@@ -545,10 +556,10 @@ int Solver::upload(int ix, const double* host, size_t n) {
         // host blocks [Ex|..|Hz] -> node-major device layout (6 values per node)
         NW_TRY_HIP(hipMemcpyAsync(d_stage, host, 8 * 6 * P, hipMemcpyHostToDevice, stream));
         if (prec == kFP64) {
-            double* dst = static_cast<double*>(d_u[cur]) + 6 * I.node_base;
+            double* dst = static_cast<double*>(d_u[parity_of(I)]) + 6 * I.node_base;
             NW_TRY_HIP((launch_convert<double, double>(dst, 1, 6, d_stage, P, 1, P, 6, stream)));
         } else {
-            float* dst = static_cast<float*>(d_u[cur]) + 6 * I.node_base;
+            float* dst = static_cast<float*>(d_u[parity_of(I)]) + 6 * I.node_base;
             NW_TRY_HIP((launch_convert<float, double>(dst, 1, 6, d_stage, P, 1, P, 6, stream)));
         }
     }
@@ -568,10 +579,10 @@ int Solver::download(int ix, double* host, size_t n) {
         NW_TRY_HIP(hipMemcpy2DAsync(host, P * 8, d_state, S * 8, P * 8, 6, hipMemcpyDeviceToHost, stream));
     } else {
         if (prec == kFP64) {
-            const double* src = static_cast<const double*>(d_u[cur]) + 6 * I.node_base;
+            const double* src = static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base;
             NW_TRY_HIP((launch_convert<double, double>(d_stage, P, 1, src, 1, 6, P, 6, stream)));
         } else {
-            const float* src = static_cast<const float*>(d_u[cur]) + 6 * I.node_base;
+            const float* src = static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base;
             NW_TRY_HIP((launch_convert<double, float>(d_stage, P, 1, src, 1, 6, P, 6, stream)));
         }
         NW_TRY_HIP(hipMemcpyAsync(host, d_stage, 8 * 6 * P, hipMemcpyDeviceToHost, stream));
@@ -638,7 +649,7 @@ int Solver::launch_segment(const Segment& sg, int s, int parity, int option, int
 
 // One stage of the fused pipeline, reading d_u[parity] and writing d_u[1-parity].
 // Segments of different n1 are independent within a stage.
-int Solver::enqueue_fused_stage(int s, int parity) {
+int Solver::enqueue_fused_stage(const StageSet& S, int s, int parity) {
     void* uin = d_u[parity];
     if (nhalo > 0) {
         const int nh = static_cast<int>(nhalo);
@@ -668,8 +679,8 @@ int Solver::enqueue_fused_stage(int s, int parity) {
     // then takes its segments in reverse order (the segment at the turn starts
     // on its own last writes)
     const bool back = parity != 0 && alternating_walk();
-    for (size_t i = 0; i < seg.size(); ++i) {
-        const size_t x = back ? seg.size() - 1 - i : i;
+    for (size_t i = 0; i < S.segs.size(); ++i) {
+        const size_t x = size_t(S.segs[back ? S.segs.size() - 1 - i : i]);
         if ((st = launch_segment(seg[x], s, parity, seg[x].option, stream_of(seg[x], seg[x].option), stream, back)))
             return st;
     }
@@ -709,10 +720,10 @@ int Solver::enqueue_plain_stage(int s) {
     return NW_OK;
 }
 
-int Solver::enqueue_step(int parity) {
+int Solver::enqueue_step(const StageSet& S, int parity) {
     int st;
     for (int s = 0; s < kStages; ++s) {
-        if (pipe == NW_PIPE_FUSED) st = enqueue_fused_stage(s, (parity + s) & 1);
+        if (pipe == NW_PIPE_FUSED) st = enqueue_fused_stage(S, s, (parity + s) & 1);
         else st = enqueue_plain_stage(s);
         if (st) return st;
     }
@@ -736,12 +747,13 @@ int Solver::enqueue_probe(int state_parity) {
 }
 
 void Solver::drop_graphs() {
-    for (int p = 0; p < 2; ++p) {
-        if (gexec[p]) (void)hipGraphExecDestroy(gexec[p]);
-        if (graph[p]) (void)hipGraphDestroy(graph[p]);
-        gexec[p] = nullptr;
-        graph[p] = nullptr;
-    }
+    for (StageSet& S : sets)
+        for (int p = 0; p < 2; ++p) {
+            if (S.gexec[p]) (void)hipGraphExecDestroy(S.gexec[p]);
+            if (S.graph[p]) (void)hipGraphDestroy(S.graph[p]);
+            S.gexec[p] = nullptr;
+            S.graph[p] = nullptr;
+        }
 }
 
 // ProbeManager::init (probe.cpp:42-103) for the device: place the probes on the
@@ -763,6 +775,12 @@ int Solver::set_probes(const Mesh& m, int n, const double* xyz, int capacity) {
     dfree(d_probe_base);
     dfree(d_probe_w);
     dfree(d_probe_hist);
+    dfree(d_snap);
+    dfree(d_snap_slot);
+    dfree(d_snap_base);
+    d_snap = nullptr;
+    d_snap_slot = nullptr;
+    d_snap_base = nullptr;
     d_probe_base = nullptr;
     d_probe_w = nullptr;
     d_probe_hist = nullptr;
@@ -782,6 +800,21 @@ int Solver::set_probes(const Mesh& m, int n, const double* xyz, int capacity) {
     if ((st = upload_vec(&d_probe_w, lw))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_probe_hist), sizeof(double) * 6 * size_t(n) * capacity))) return st;
     if (!d_probe_slot && (st = dalloc(reinterpret_cast<void**>(&d_probe_slot), sizeof(int)))) return st;
+    if (!sets[1].segs.empty()) {  // the probed elements' slots in a resident launch's snapshots
+        std::vector<int> slot(static_cast<size_t>(nelt), -1);
+        std::vector<long long> sbase(n);
+        snap_slots = 0;
+        for (int q = 0; q < n; ++q) {
+            int& s = slot[size_t(elem[q])];
+            if (s < 0) s = snap_slots++;
+            sbase[q] = (long long)s * 6 * np;
+        }
+        const long long bytes = (long long)snap_slots * 6 * np * (prec == kFP64 ? 8 : 4);
+        snap_steps = static_cast<int>(std::max(1ll, std::min<long long>(capacity, kSnapBytes / bytes)));
+        if ((st = upload_vec(&d_snap_slot, slot))) return st;
+        if ((st = upload_vec(&d_snap_base, sbase))) return st;
+        if ((st = dalloc(&d_snap, size_t(bytes) * size_t(snap_steps)))) return st;
+    }
     NW_TRY_HIP(launch_zero_int(d_probe_slot, stream));
     NW_TRY_HIP(hipStreamSynchronize(stream));
     nprobes = n;
@@ -795,7 +828,7 @@ int Solver::probe_sample() {
     if (!initialized || !uploaded) { set_error("probe_sample before create/upload"); return NW_ERR_STATE; }
     if (nprobes <= 0) { set_error("no probes set"); return NW_ERR_STATE; }
     NW_TRY_HIP(hipSetDevice(device));
-    int st = enqueue_probe(cur);
+    int st = enqueue_probe(pipe == NW_PIPE_FUSED ? parity_of(inst[0]) : 0);
     if (st) return st;
     NW_TRY_HIP(hipStreamSynchronize(stream));
     return NW_OK;
@@ -827,10 +860,10 @@ int Solver::probe_history(double* host, int max_records, int* nrecords) {
     return NW_OK;
 }
 
-int Solver::build_graph(int parity) {
+int Solver::build_graph(StageSet& S, int parity) {
     hipGraph_t g = nullptr;
     NW_TRY_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-    int st = enqueue_step(parity);
+    int st = enqueue_step(S, parity);
     hipError_t e = hipStreamEndCapture(stream, &g);
     if (st) {
         if (g) (void)hipGraphDestroy(g);
@@ -847,8 +880,8 @@ int Solver::build_graph(int parity) {
         set_error(std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
         return NW_ERR_HIP;
     }
-    graph[parity] = g;
-    gexec[parity] = x;
+    S.graph[parity] = g;
+    S.gexec[parity] = x;
     return NW_OK;
 }
 
@@ -882,13 +915,18 @@ std::map<TuneKey, std::pair<int, int>> g_tune;  // (tile option, non-temporal k)
 // read k) and keep the fastest.  The options alternate twice and each keeps its
 // best time, so a slow moment of the GPU does not decide.  Runs at a step
 // boundary, before graphs are captured.
-int Solver::tune() {
+int Solver::tune() { return tune_segments(true); }
+
+// all: every segment; else those that only the staged launches run.
+int Solver::tune_segments(bool all) {
     if (pipe != NW_PIPE_FUSED) return NW_OK;
     NW_TRY_HIP(hipSetDevice(device));
     // non-temporal k is a candidate only where the working set exceeds the
     // Infinity Cache (below it the hint only costs)
     const int nstream = fused_beyond_infinity_cache(working_set_bytes()) ? 2 : 1;
     for (Segment& sg : seg) {
+        if (!all && !sg.parts.empty()) continue;
+        const int cur = sets[sg.parts.empty() ? 0 : 1].cur;
         const TuneKey key{device, sg.n1, prec, inst.size() == 1 ? 1 : 0, nstream - 1, groups_per_cu, sg.nelt};
         {
             std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -969,6 +1007,7 @@ int Solver::set_segment_option(int s, int option, int stream_k) {
     seg[size_t(s)].option = option;
     seg[size_t(s)].stream = stream_k;
     tuned = true;  // an explicit choice stands until tune() is called
+    staged_only = true;
     drop_graphs();
     return NW_OK;
 }
@@ -991,7 +1030,26 @@ int Solver::set_walk(int mode) {
     NW_TRY_HIP(hipSetDevice(device));
     NW_TRY_HIP(hipStreamSynchronize(stream));
     walk_mode = mode;
+    if (mode >= 0) staged_only = true;
     drop_graphs();  // captured launches carry the previous direction
+    return NW_OK;
+}
+
+// nsteps steps of one set by stage launches (plain pipeline: sets[0], no segments used).
+int Solver::enqueue_staged(StageSet& S, double dt, int nsteps) {
+    if (nsteps <= 0) return NW_OK;
+    int st = set_dt(dt);
+    if (st) return st;
+    for (int n = 0; n < nsteps; ++n) {
+        const int parity = (pipe == NW_PIPE_FUSED) ? S.cur : 0;
+        if (use_graph) {
+            if (!S.gexec[parity] && (st = build_graph(S, parity))) return st;
+            NW_TRY_HIP(hipGraphLaunch(S.gexec[parity], stream));
+        } else {
+            if ((st = enqueue_step(S, parity))) return st;
+        }
+        if (pipe == NW_PIPE_FUSED) S.cur ^= 1;  // five stages flip the ping-pong parity
+    }
     return NW_OK;
 }
 
@@ -1000,40 +1058,39 @@ int Solver::launch_steps(double dt, int nsteps) {
     if (!uploaded) { set_error("step before uploadState"); return NW_ERR_STATE; }
     NW_CHECK_ARG(nsteps >= 0, "nsteps must be >= 0");
     NW_TRY_HIP(hipSetDevice(device));
-    int st = set_dt(dt);
-    if (st) return st;
-    if (autotune && !tuned && nsteps > 0 && (st = tune())) return st;
-    for (int n = 0; n < nsteps; ++n) {
-        const int parity = (pipe == NW_PIPE_FUSED) ? cur : 0;
-        if (use_graph) {
-            if (!gexec[parity] && (st = build_graph(parity))) return st;
-            NW_TRY_HIP(hipGraphLaunch(gexec[parity], stream));
-        } else {
-            if ((st = enqueue_step(parity))) return st;
-        }
-        if (pipe == NW_PIPE_FUSED) cur ^= 1;  // five stages flip the ping-pong parity
-    }
+    if (nsteps == 0) return NW_OK;
+    int st;
+    const bool resident = hold_resident();
+    if (autotune && !tuned && !sets[0].segs.empty() && (st = tune_segments(false))) return st;
+    if (resident && (st = enqueue_resident(dt, nsteps))) return st;
+    for (int x = 0; x < 2; ++x)
+        if (!sets[x].segs.empty() && !(x == 1 && resident) && (st = enqueue_staged(sets[x], dt, nsteps))) return st;
     return NW_OK;
 }
 
 int Solver::step(double dt, int nsteps) {
-    int st = launch_steps(dt, nsteps);
-    if (st) return st;
-    NW_TRY_HIP(hipStreamSynchronize(stream));
-    return NW_OK;
+    const int st = launch_steps(dt, nsteps);
+    const int fin = finish();
+    return st ? st : fin;
 }
 
 int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
     if (!initialized || !uploaded) { set_error("time before create/upload"); return NW_ERR_STATE; }
     NW_CHECK_ARG(warmup >= 0 && nsteps >= 0 && repeats >= 1 && repeats <= 1024, "bad warmup/steps/repeats");
     NW_TRY_HIP(hipSetDevice(device));
-    int st = set_dt(dt);
-    if (st) return st;
+    int st;
     // tune and capture outside the timed region
-    if (autotune && !tuned && (st = tune())) return st;
+    const bool resident = hold_resident();
+    if (autotune && !tuned && !sets[0].segs.empty() && (st = tune_segments(false))) { finish(); return st; }
     if (use_graph) {
-        for (int p = 0; p < 2; ++p)
-            if (!gexec[p] && (pipe == NW_PIPE_FUSED || p == 0) && (st = build_graph(p))) return st;
+        if ((st = set_dt(dt))) { finish(); return st; }
+        for (int x = 0; x < 2; ++x)
+            for (int p = 0; p < 2; ++p)
+                if (!sets[x].segs.empty() && !(x == 1 && resident) && !sets[x].gexec[p] &&
+                    (pipe == NW_PIPE_FUSED || p == 0) && (st = build_graph(sets[x], p))) {
+                    finish();
+                    return st;
+                }
     }
     // warm-up steps, then `repeats` timed runs of exactly nsteps steps, all
     // queued back to back: no host wait between them, one at the end
@@ -1046,18 +1103,19 @@ int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
         const hipError_t he = hipEventCreate(&e);
         if (he != hipSuccess) {
             destroy();
+            finish();
             set_error(std::string("hipEventCreate: ") + hipGetErrorString(he));
             return NW_ERR_HIP;
         }
     }
     hipError_t he = hipSuccess;
-    if ((st = launch_steps(dt, warmup))) { destroy(); return st; }
-    he = hipEventRecord(ev[0], stream);
+    if ((st = launch_steps(dt, warmup)) == NW_OK) he = hipEventRecord(ev[0], stream);
     for (int r = 0; r < repeats && he == hipSuccess && st == NW_OK; ++r) {
         st = launch_steps(dt, nsteps);
         if (st == NW_OK) he = hipEventRecord(ev[size_t(r) + 1], stream);
     }
-    if (he == hipSuccess && st == NW_OK) he = hipEventSynchronize(ev[size_t(repeats)]);
+    const int fin = finish();
+    if (st == NW_OK) st = fin;
     for (int r = 0; r < repeats && he == hipSuccess && st == NW_OK; ++r) {
         float f = 0.0f;
         he = hipEventElapsedTime(&f, ev[size_t(r)], ev[size_t(r) + 1]);
@@ -1072,6 +1130,169 @@ int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
     return NW_OK;
 }
 
+// ---------------------------------------------------------------------------
+// resident launches
+// ---------------------------------------------------------------------------
+namespace {
+// One resident launch at a time per device in this process: its workgroups wait
+// for each other, so two such grids that each hold part of the CUs would wait
+// until their polls run out.  Another solver's call meanwhile takes the staged
+// launches, which wait for nothing.
+std::atomic<bool> g_resident_busy[64];
+}  // namespace
+
+bool Solver::hold_resident() {
+    if (staged_only || sets[1].segs.empty()) return false;
+    if (!resident_held) resident_held = !g_resident_busy[device].exchange(true, std::memory_order_acquire);
+    return resident_held;
+}
+
+void Solver::release_resident() {
+    if (resident_held) g_resident_busy[device].store(false, std::memory_order_release);
+    resident_held = false;
+}
+
+// The meshes of each segment that fit on chip, cut into launches of whole
+// meshes; the tables and buffers of those launches.  A segment takes resident
+// launches wherever all its meshes fit: measured faster at every size up to the
+// chip's (nw_resident_kernel.hpp), by least at the largest (n1 = 8, 1728 jittered
+// elements: 1.28x).  The smallest kernel size that holds a launch is taken (more
+// workgroups per CU to overlap; n1 = 8, 1000 elements: two per workgroup 8.8 us per
+// stage, four 10.9).  Not with explicit launch shapes (tile option, segment choice,
+// walk), ghost faces or split BF16.  NW_RESIDENT=0: stage launches only (the two
+// give the same bits; tests compare them).
+int Solver::init_resident(const Mesh* const* meshes) {
+    const char* env = std::getenv("NW_RESIDENT");
+    if (!autotune || prec == kBF16X3 || nhalo > 0 || device >= 64 || (env && env[0] == '0')) return NW_OK;
+    std::vector<int4> nbr(size_t(nelt) * 6, make_int4(-1, 0, 0, 0));
+    std::vector<int> order(inst.size());
+    std::iota(order.begin(), order.end(), 0);
+    std::sort(order.begin(), order.end(), [&](int a, int b) { return inst[size_t(a)].elem_base < inst[size_t(b)].elem_base; });
+    long long bytes = 0;
+    for (size_t si = 0; si < seg.size(); ++si) {
+        Segment& sg = seg[si];
+        long long cap[kResidentSizes], most = 0;
+        for (int em = 0; em < kResidentSizes; ++em) {
+            cap[em] = resident_capacity(sg.n1, prec, em, sg.affine, groups_per_cu);
+            most = std::max(most, cap[em]);
+        }
+        std::vector<ResidentPart> parts;
+        bool fits = true;
+        for (int r : order) {
+            const Instance& I = inst[size_t(r)];
+            if (I.seg != static_cast<int>(si) || !fits) continue;
+            const int e0 = I.elem_base - sg.elem_base;
+            fits = I.nelt <= most && resident_face_table(meshes[r]->fcode.data(), I.nelt, I.n1, e0, &nbr[size_t(I.elem_base) * 6]);
+            if (parts.empty() || parts.back().nelt + I.nelt > most) parts.push_back({e0});
+            parts.back().nelt += I.nelt;
+        }
+        if (!fits) continue;
+        for (ResidentPart& P : parts) {
+            while (cap[P.em] < P.nelt) ++P.em;
+            const long long groups = cap[P.em] / resident_em(P.em);
+            P.per = static_cast<int>((P.nelt + groups - 1) / groups);
+            bytes = std::max(bytes, resident_xchg_bytes(sg.n1, prec, P.nelt));
+        }
+        sg.parts = parts;
+    }
+    if (bytes == 0) return NW_OK;
+    int st;
+    if ((st = upload_vec(&d_rnbr, nbr))) return st;
+    if ((st = dalloc(reinterpret_cast<void**>(&d_xchg), size_t(bytes)))) return st;
+    if ((st = dalloc(reinterpret_cast<void**>(&d_stop), sizeof(int)))) return st;
+    NW_TRY_HIP(hipMemsetAsync(d_xchg, 0, size_t(bytes), stream));  // no tag matches an epoch that has not been stored
+    NW_TRY_HIP(hipMemsetAsync(d_stop, 0, sizeof(int), stream));
+    NW_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_stop), sizeof(int), hipHostMallocDefault));
+    *h_stop = 0;
+    return NW_OK;
+}
+
+int Solver::enqueue_resident(double dt, int nsteps) {
+    const size_t rsz = prec == kFP64 ? 8 : 4;
+    const char* env = std::getenv("NW_RESIDENT_SPINS");  // a test's bound on the kernel's own waits
+    StageSet& S = sets[1];
+    resident_dt = dt;
+    while (nsteps > 0) {
+        const int n = std::min(nsteps, nprobes > 0 ? std::min(kResidentSteps, snap_steps) : kResidentSteps);
+        resident_log.push_back({resident_seq + 1, S.cur, n});
+        for (int x : S.segs) {
+            const Segment& sg = seg[size_t(x)];
+            for (const ResidentPart& P : sg.parts) {
+                ResidentArgs a{};
+                a.uin = d_u[S.cur];
+                a.uout = d_u[1 - S.cur];
+                a.rec = d_rec + size_t(sg.elem_base) * 26;
+                a.fw = static_cast<const char*>(d_fw) + size_t(sg.elem_base) * 24 * rsz;
+                a.nbr = d_rnbr + size_t(sg.elem_base) * 6;
+                a.xchg = d_xchg;
+                a.snap = nprobes > 0 ? d_snap : nullptr;
+                a.snap_slot = d_snap_slot;
+                a.nslots = snap_slots;
+                a.node_base = sg.node_base;
+                a.elem0 = P.elem0;
+                a.nelt = P.nelt;
+                a.per = P.per;
+                a.nsteps = n;
+                a.epoch = resident_epoch;
+                a.stop = d_stop;
+                a.stop_host = h_stop;
+                a.seq = ++resident_seq;
+                a.spin_limit = env ? std::atoi(env) : 1 << 20;
+                a.dt = dt;
+                for (int s = 0; s < kStages; ++s) {
+                    a.a[s] = kRkA[s];
+                    a.b[s] = kRkB[s];
+                }
+                resident_epoch += 5u * static_cast<unsigned>(n);
+                NW_TRY_HIP(launch_resident(sg.n1, prec, P.em, sg.affine, a, stream));
+            }
+        }
+        S.cur ^= 1;  // a launch reads one buffer and writes the other, whatever its steps
+        if (nprobes > 0) {
+            const long long per_step = (long long)snap_slots * 6 * np;
+            if (prec == kFP64)
+                NW_TRY_HIP(launch_probe<double>(static_cast<const double*>(d_snap), np, 1, nprobes, d_snap_base, d_probe_w, n1,
+                                                d_probe_hist, d_probe_slot, probe_cap, stream, n, per_step, d_stop));
+            else
+                NW_TRY_HIP(launch_probe<float>(static_cast<const float*>(d_snap), np, 1, nprobes, d_snap_base, d_probe_w, n1,
+                                               d_probe_hist, d_probe_slot, probe_cap, stream, n, per_step, d_stop));
+        }
+        nsteps -= n;
+    }
+    return NW_OK;
+}
+
+// Waits for the stream.  Where a resident launch gave up (its workgroups were not
+// all placed, another process holding the GPU), its input buffer is as it was
+// and later launches left everything alone: the steps from there on are run
+// again by stage launches, and this solver keeps to those.
+int Solver::finish() {
+    if (!initialized) return NW_OK;
+    hipError_t he = hipStreamSynchronize(stream);
+    int st = NW_OK;
+    if (he == hipSuccess && !resident_log.empty() && *static_cast<volatile int*>(h_stop) != 0) {
+        const int seq = *static_cast<volatile int*>(h_stop);
+        size_t c = resident_log.size() - 1;
+        while (c > 0 && resident_log[c].seq > seq) --c;
+        int left = 0;
+        for (size_t x = c; x < resident_log.size(); ++x) left += resident_log[x].steps;
+        sets[1].cur = resident_log[c].cur;
+        staged_only = true;
+        *h_stop = 0;
+        he = hipMemset(d_stop, 0, sizeof(int));
+        if (he == hipSuccess) st = enqueue_staged(sets[1], resident_dt, left);
+        if (he == hipSuccess) he = hipStreamSynchronize(stream);
+    }
+    resident_log.clear();
+    resident_seq = 0;
+    release_resident();
+    if (he != hipSuccess) {
+        set_error(std::string("hipStreamSynchronize: ") + hipGetErrorString(he));
+        return NW_ERR_HIP;
+    }
+    return st;
+}
+
 int Solver::diag(int ix, nw_diag* out) {
     if (!initialized) { set_error("diag before create"); return NW_ERR_STATE; }
     NW_CHECK_ARG(ix >= 0 && ix < (int)inst.size(), "bad instance index");
@@ -1083,10 +1304,10 @@ int Solver::diag(int ix, nw_diag* out) {
         NW_TRY_HIP(launch_diag<double>(d_state, stride, 1, npts, n1, d_met[3], nullptr, mat, d_diag_part, d_diag_out,
                                        stream));
     } else if (prec == kFP64) {
-        NW_TRY_HIP(launch_diag<double>(static_cast<const double*>(d_u[cur]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
+        NW_TRY_HIP(launch_diag<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
                                        nullptr, geom, mat, d_diag_part, d_diag_out, stream));
     } else {
-        NW_TRY_HIP(launch_diag<float>(static_cast<const float*>(d_u[cur]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
+        NW_TRY_HIP(launch_diag<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
                                       nullptr, geom, mat, d_diag_part, d_diag_out, stream));
     }
     double h[3];
@@ -1113,10 +1334,10 @@ int Solver::rel_l2(int ix, const double* ref, size_t n, double* out) {
         NW_TRY_HIP(launch_l2<double>(d_state, stride, 1, d_stage, npts, n1, d_met[3], nullptr, d_diag_part, d_diag_out,
                                      stream));
     } else if (prec == kFP64) {
-        NW_TRY_HIP(launch_l2<double>(static_cast<const double*>(d_u[cur]) + 6 * I.node_base, 1, 6, d_stage, I.npts,
+        NW_TRY_HIP(launch_l2<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts,
                                      I.n1, nullptr, geom, d_diag_part, d_diag_out, stream));
     } else {
-        NW_TRY_HIP(launch_l2<float>(static_cast<const float*>(d_u[cur]) + 6 * I.node_base, 1, 6, d_stage, I.npts, I.n1,
+        NW_TRY_HIP(launch_l2<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts, I.n1,
                                     nullptr, geom, d_diag_part, d_diag_out, stream));
     }
     double h[2];

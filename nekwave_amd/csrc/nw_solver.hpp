@@ -6,6 +6,7 @@
 
 #include "nw_fused.hpp"
 #include "nw_mesh.hpp"
+#include "nw_resident.hpp"
 
 namespace nw {
 
@@ -14,6 +15,13 @@ struct Instance {
     int n1 = 0, np = 0, nelt = 0, elem_base = 0;
     long long node_base = 0, npts = 0;
     bool media = false;
+    int seg = 0;  // the segment that holds it
+};
+
+// Elements that one launch of the resident kernel keeps on chip: whole meshes of
+// one segment, `per` elements per workgroup of the kernel size `em`.
+struct ResidentPart {
+    int elem0 = 0, nelt = 0, per = 0, em = 0;
 };
 
 // A run of elements sharing n1: one fused launch per stage.
@@ -26,6 +34,17 @@ struct Segment {
     long long goff[kNumTileOptions] = {};  // offset of this segment's group order, per tile option
     long long soff[kNumTileOptions] = {};  // offset of its workgroup sequence offsets, per tile option
     int nseq[kNumTileOptions] = {};        // its workgroup sequences, per tile option
+    std::vector<ResidentPart> parts;       // resident launches that cover it (empty: staged only)
+};
+
+// Segments that advance together: one ping-pong parity and one graph per parity.
+// Set 0: segments that only the staged launches run; set 1: segments that fit on
+// chip, which the staged launches run where the resident kernel may not.
+struct StageSet {
+    std::vector<int> segs;
+    int cur = 0;  // d_u[cur] holds the set's state
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t gexec[2] = {nullptr, nullptr};
 };
 
 // FNV-1a hash of what makes a mesh this mesh: n1, corner coordinates (bit
@@ -46,7 +65,7 @@ struct Solver {
     long long npts = 0, tfp = 0, nhalo = 0, stride = 0, device_bytes = 0;
     long long kchunks = 0;  // fused pipeline: k chunks of 6 x 64 values (Segment::kbase)
     double c0 = 1.0, last_dt = -1.0;
-    int cur = 0;
+    StageSet sets[2];
     std::vector<Instance> inst;  // in caller order
     std::vector<Segment> seg;
     std::vector<void*> allocs;
@@ -72,6 +91,24 @@ struct Solver {
     int* d_ghead = nullptr;   // per segment and tile option: kFusedHead words per workgroup sequence
     int* d_gorder_rev = nullptr;  // the same walks with every sequence visited backwards
     int* d_ghead_rev = nullptr;
+    // resident launches (sets[1])
+    bool staged_only = false;  // explicit launch shapes were asked for, or a resident launch gave up
+    bool resident_held = false;  // this solver has the device's resident slot
+    int resident_seq = 0;        // launches since the last finish()
+    unsigned resident_epoch = 1;
+    double resident_dt = 0.0;
+    struct ResidentChunk {
+        int seq, cur, steps;  // first launch, input parity, steps
+    };
+    std::vector<ResidentChunk> resident_log;
+    int4* d_rnbr = nullptr;
+    unsigned long long* d_xchg = nullptr;
+    int* d_stop = nullptr;
+    int* h_stop = nullptr;  // host memory the kernel writes
+    void* d_snap = nullptr;        // probed elements' fields after each step of a launch
+    int* d_snap_slot = nullptr;    // per element: its slot in d_snap, -1 none
+    long long* d_snap_base = nullptr;  // per probe: its element's offset in a step's record
+    int snap_slots = 0, snap_steps = 0;
     // plain pipeline (reference residency, single mesh)
     double *d_state = nullptr, *d_kk = nullptr, *d_rhs = nullptr, *d_D = nullptr, *d_w3 = nullptr;
     double* d_met[13] = {};  // x y z jac rx sx tx ry sy ty rz sz tz
@@ -85,9 +122,6 @@ struct Solver {
     double* d_probe_w = nullptr;
     double* d_probe_hist = nullptr;
     int* d_probe_slot = nullptr;
-    // graphs per starting parity
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t gexec[2] = {nullptr, nullptr};
 
     ~Solver();
     void release();
@@ -103,6 +137,7 @@ struct Solver {
     int probe_sample();
     int probe_history(double* host, int max_records, int* nrecords);
     int tune();
+    int finish();  // waits for the stream; a resident launch that gave up is run again staged
     int set_segment_option(int s, int option, int stream_k);
     int set_walk(int mode);  // -1 auto (fused_alternate_walk), 0 forwards, 1 alternating
     bool alternating_walk() const;
@@ -117,13 +152,21 @@ struct Solver {
     int upload_vec(T** dst, const std::vector<T>& v);
     int init_plain(const Mesh& m);
     int set_dt(double dt);
+    int set_of(int segment) const { return seg[size_t(segment)].parts.empty() ? 0 : 1; }
+    int parity_of(const Instance& I) const { return sets[set_of(I.seg)].cur; }
+    int init_resident(const Mesh* const* meshes);
+    int tune_segments(bool all);
+    int enqueue_staged(StageSet& S, double dt, int nsteps);
+    int enqueue_resident(double dt, int nsteps);
+    bool hold_resident();
+    void release_resident();
     int launch_segment(const Segment& sg, int s, int parity, int option, int stream_k, hipStream_t st,
                        bool backwards = false);
     long long working_set_bytes() const;
-    int enqueue_fused_stage(int s, int parity);
+    int enqueue_fused_stage(const StageSet& S, int s, int parity);
     int enqueue_plain_stage(int s);
-    int enqueue_step(int parity);
-    int build_graph(int parity);
+    int enqueue_step(const StageSet& S, int parity);
+    int build_graph(StageSet& S, int parity);
     int enqueue_probe(int state_parity);
     void drop_graphs();
 };
