@@ -413,13 +413,29 @@ __global__ void k_diag_partial(const R* __restrict__ u, long long cs, long long 
     }
 }
 
-__global__ void k_diag_final(const double* __restrict__ part, int n, double* __restrict__ out) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double en = 0.0, me = 0.0, mh = 0.0;
-        for (int b = 0; b < n; ++b) {
-            en += part[3 * b]; me = fmax(me, part[3 * b + 1]); mh = fmax(mh, part[3 * b + 2]);
+// The partial triples of the blocks, reduced by one workgroup: kFinal threads stride
+// over them, then a tree in LDS.  (One thread walking 1024 triples was a serial chain
+// of dependent additions and reads: 121 us; this 4 us, most of it the launch.)
+constexpr int kFinal = 256;
+__global__ __launch_bounds__(kFinal) void k_diag_final(const double* __restrict__ part, int n, double* __restrict__ out) {
+    __shared__ double sh[3][kFinal];
+    const int t = threadIdx.x;
+    double en = 0.0, me = 0.0, mh = 0.0;
+    for (int b = t; b < n; b += kFinal) {
+        en += part[3 * b]; me = fmax(me, part[3 * b + 1]); mh = fmax(mh, part[3 * b + 2]);
+    }
+    sh[0][t] = en; sh[1][t] = me; sh[2][t] = mh;
+    __syncthreads();
+    for (int w = kFinal / 2; w > 0; w >>= 1) {
+        if (t < w) {
+            sh[0][t] += sh[0][t + w];
+            sh[1][t] = fmax(sh[1][t], sh[1][t + w]);
+            sh[2][t] = fmax(sh[2][t], sh[2][t + w]);
         }
-        out[0] = en; out[1] = sqrt(me); out[2] = sqrt(mh);
+        __syncthreads();
+    }
+    if (t == 0) {
+        out[0] = sh[0][0]; out[1] = sqrt(sh[1][0]); out[2] = sqrt(sh[2][0]);
     }
 }
 
@@ -501,13 +517,24 @@ __global__ void k_l2_partial(const R* __restrict__ u, long long cs, long long ns
     }
 }
 
-__global__ void k_l2_final(const double* __restrict__ part, int n, double* __restrict__ out) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        double num = 0.0, den = 0.0;
-        for (int b = 0; b < n; ++b) {
-            num += part[2 * b]; den += part[2 * b + 1];
+__global__ __launch_bounds__(kFinal) void k_l2_final(const double* __restrict__ part, int n, double* __restrict__ out) {
+    __shared__ double sh[2][kFinal];
+    const int t = threadIdx.x;
+    double num = 0.0, den = 0.0;
+    for (int b = t; b < n; b += kFinal) {
+        num += part[2 * b]; den += part[2 * b + 1];
+    }
+    sh[0][t] = num; sh[1][t] = den;
+    __syncthreads();
+    for (int w = kFinal / 2; w > 0; w >>= 1) {
+        if (t < w) {
+            sh[0][t] += sh[0][t + w];
+            sh[1][t] += sh[1][t + w];
         }
-        out[0] = num; out[1] = den;
+        __syncthreads();
+    }
+    if (t == 0) {
+        out[0] = sh[0][0]; out[1] = sh[1][0];
     }
 }
 
@@ -726,7 +753,7 @@ hipError_t launch_diag(const R* u, long long cs, long long ns, long long npts, i
                        const ElemGeom* geom, const ElemMat* mat, double* part, double* out, hipStream_t s) {
     const int nb = diag_blocks();
     hipLaunchKernelGGL(k_diag_partial<R>, dim3(nb), dim3(kBlock), 0, s, u, cs, ns, npts, n1, jac, geom, mat, part);
-    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64), 0, s, part, nb, out);
+    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(kFinal), 0, s, part, nb, out);
     return hipGetLastError();
 }
 // Partial sums of nw_launch_diagnostics_noalloc: a fixed device array (one
@@ -761,7 +788,7 @@ hipError_t launch_energy(const double* st, long long S, long long npts, int n1, 
                          const double* eps, const double* mu, double* part, double* out, hipStream_t s) {
     const int nb = energy_blocks(npts);
     hipLaunchKernelGGL(k_energy_partial, dim3(nb), dim3(kBlock), 0, s, st, S, npts, n1, jac, w, eps, mu, part);
-    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(64), 0, s, part, nb, out);
+    hipLaunchKernelGGL(k_diag_final, dim3(1), dim3(kFinal), 0, s, part, nb, out);
     return hipGetLastError();
 }
 
@@ -770,7 +797,7 @@ hipError_t launch_l2(const R* u, long long cs, long long ns, const double* ref, 
                      const ElemGeom* geom, double* part, double* out, hipStream_t s) {
     const int nb = diag_blocks();
     hipLaunchKernelGGL(k_l2_partial<R>, dim3(nb), dim3(kBlock), 0, s, u, cs, ns, ref, npts, n1, jac, geom, part);
-    hipLaunchKernelGGL(k_l2_final, dim3(1), dim3(64), 0, s, part, nb, out);
+    hipLaunchKernelGGL(k_l2_final, dim3(1), dim3(kFinal), 0, s, part, nb, out);
     return hipGetLastError();
 }
 template hipError_t launch_l2<double>(const double*, long long, long long, const double*, long long, int, const double*,

@@ -55,7 +55,7 @@ hipError_t launch_diag(const R* u, long long cs, long long ns, long long npts, i
 // Energy, max |E|, max |H| of a reference-layout FP64 state into out[0..2]
 // (Case::computeTotalEnergy / getMaxE / getMaxH, case.cpp:733-794): one partial
 // triple per block into part (3 energy_blocks(npts) doubles, every one written,
-// none read before), then one reduction in block order.
+// none read before), then one workgroup reduces them (a fixed tree).
 constexpr int kEnergyMaxBlocks = 1024;
 int energy_blocks(long long npts);
 // The device address of this GPU's fixed partial-sum array (3 kEnergyScratchBlocks
