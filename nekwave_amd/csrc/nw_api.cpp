@@ -249,20 +249,28 @@ NW_API int nw_batch_create(int count, const nw_mesh* const* meshes, double c0, c
 }
 
 NW_API int nw_dg_upload(nw_dg* s, const double* host, size_t n) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.upload(0, host, n);
+    NW_GUARD_END
 }
 NW_API int nw_dg_download(nw_dg* s, double* host, size_t n) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.download(0, host, n);
+    NW_GUARD_END
 }
 NW_API int nw_dg_upload_instance(nw_dg* s, int instance, const double* host, size_t n) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.upload(instance, host, n);
+    NW_GUARD_END
 }
 NW_API int nw_dg_download_instance(nw_dg* s, int instance, double* host, size_t n) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.download(instance, host, n);
+    NW_GUARD_END
 }
 NW_API int nw_dg_rel_l2(nw_dg* s, int instance, const double* ref, size_t n, double* rel_l2) {
     NW_CHECK_ARG(s, "null solver");
@@ -279,8 +287,10 @@ NW_API int nw_dg_probe_sample(nw_dg* s) {
     return s->s.probe_sample();
 }
 NW_API int nw_dg_probe_history(nw_dg* s, double* out, int max_records, int* nrecords) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.probe_history(out, max_records, nrecords);
+    NW_GUARD_END
 }
 NW_API int nw_mesh_locate_probes(const nw_mesh* m, int n, const double* xyz, int* elem, double* rst) {
     NW_CHECK_ARG(m && n >= 0 && (n == 0 || (xyz && elem && rst)), "null argument");
@@ -292,12 +302,14 @@ NW_API int nw_dg_diag_instance(nw_dg* s, int instance, nw_diag* out) {
     return s->s.diag(instance, out);
 }
 NW_API int nw_dg_tune(nw_dg* s) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     if (!s->s.uploaded) {
         nw::set_error("tune needs an uploaded state");
         return NW_ERR_STATE;
     }
     return s->s.tune();
+    NW_GUARD_END
 }
 NW_API int nw_dg_set_segment_option(nw_dg* s, int seg, int option, int stream_k) {
     NW_CHECK_ARG(s, "null solver");
@@ -330,21 +342,29 @@ NW_API int nw_dg_segment_option(const nw_dg* s, int seg, int* option, int* matri
     return NW_OK;
 }
 NW_API int nw_dg_step(nw_dg* s, double dt, double time) {
+    NW_GUARD_BEGIN
     (void)time;
     NW_CHECK_ARG(s, "null solver");
     return s->s.step(dt, 1);
+    NW_GUARD_END
 }
 NW_API int nw_dg_run(nw_dg* s, double dt, int nsteps) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s, "null solver");
     return s->s.step(dt, nsteps);
+    NW_GUARD_END
 }
 NW_API int nw_dg_time(nw_dg* s, double dt, int nsteps, double* ms) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s && ms, "null argument");
     return s->s.time(dt, 0, nsteps, 1, ms);
+    NW_GUARD_END
 }
 NW_API int nw_dg_time_repeats(nw_dg* s, double dt, int warmup, int nsteps, int repeats, double* ms) {
+    NW_GUARD_BEGIN
     NW_CHECK_ARG(s && ms, "null argument");
     return s->s.time(dt, warmup, nsteps, repeats, ms);
+    NW_GUARD_END
 }
 NW_API int nw_dg_sync(nw_dg* s) {
     NW_CHECK_ARG(s, "null solver");

@@ -10,6 +10,7 @@
 //   * lift: one thread per node gathering its face contributions in face order
 //     0..5 (deterministic; the reference uses FP64 atomics, dg_kernels.cu:329);
 //   * elementwise kernels are grid-stride loops sized for 256 CUs.
+#include <algorithm>
 #include <mutex>
 
 #include "nw_plain.hpp"
@@ -600,13 +601,27 @@ __global__ void k_zero_int(int* p) {
 // ---------------------------------------------------------------------------
 // conversions and plain copy (HBM calibration)
 // ---------------------------------------------------------------------------
-template <typename D, typename S>
-__global__ void k_convert(D* __restrict__ dst, long long dcs, long long dns, const S* __restrict__ src, long long scs,
-                          long long sns, long long n, int ncomp) {
-    const long long tot = n * ncomp;
-    for (long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x < tot; x += (long long)gridDim.x * blockDim.x) {
-        const long long c = x / n, p = x - c * n;
-        dst[c * dcs + p * dns] = static_cast<D>(src[c * scs + p * sns]);
+// Nodes p0 .. p0 + n - 1 of a device state (component c of node p at c cs + p ns) from
+// a pinned host slot of six blocks of n doubles, or to one of six blocks of n device
+// values: the slot's side is coalesced and crosses the link once; bound by the link
+// (55 GB/s).  Rounding to FP32 is done here on the way in: on the host, values below
+// FP32's normal range take an assist each (12.6 MB of a pulse: 3.4 ms instead of 0.3).
+template <typename R>
+__global__ void k_state_in(R* __restrict__ u, long long cs, long long ns, long long p0, long long n,
+                           const double* __restrict__ slot) {
+    for (long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x < n; x += (long long)gridDim.x * blockDim.x) {
+        R* q = u + (p0 + x) * ns;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) q[c * cs] = static_cast<R>(slot[c * n + x]);
+    }
+}
+template <typename R>
+__global__ void k_state_out(const R* __restrict__ u, long long cs, long long ns, long long p0, long long n,
+                            R* __restrict__ slot) {
+    for (long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x < n; x += (long long)gridDim.x * blockDim.x) {
+        const R* q = u + (p0 + x) * ns;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) slot[c * n + x] = q[c * cs];
     }
 }
 
@@ -809,22 +824,25 @@ template hipError_t launch_diag<double>(const double*, long long, long long, lon
 template hipError_t launch_diag<float>(const float*, long long, long long, long long, int, const double*, const ElemGeom*,
                                        const ElemMat*, double*, double*, hipStream_t);
 
-template <typename D, typename S>
-hipError_t launch_convert(D* dst, long long dcs, long long dns, const S* src, long long scs, long long sns, long long n,
-                          int ncomp, hipStream_t s) {
+static dim3 state_grid(long long n) { return dim3(static_cast<unsigned>(std::min<long long>(256, (n + kBlock - 1) / kBlock))); }
+template <typename R>
+hipError_t launch_state_in(R* u, long long cs, long long ns, long long p0, long long n, const double* slot, hipStream_t s) {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_convert<D, S>), dim3(grid_for(n * ncomp)), dim3(kBlock), 0, s, dst, dcs, dns, src, scs, sns, n,
-                       ncomp);
+    hipLaunchKernelGGL(k_state_in<R>, state_grid(n), dim3(kBlock), 0, s, u, cs, ns, p0, n, slot);
     return hipGetLastError();
 }
-#define NW_CONVERT(D, S)                                                                                        \
-    template hipError_t launch_convert<D, S>(D*, long long, long long, const S*, long long, long long, long long, int, \
-                                             hipStream_t);
-NW_CONVERT(float, double)
-NW_CONVERT(double, float)
-NW_CONVERT(double, double)
-NW_CONVERT(float, float)
-#undef NW_CONVERT
+template <typename R>
+hipError_t launch_state_out(const R* u, long long cs, long long ns, long long p0, long long n, R* slot, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_state_out<R>, state_grid(n), dim3(kBlock), 0, s, u, cs, ns, p0, n, slot);
+    return hipGetLastError();
+}
+#define NW_STATE_MOVE(R)                                                                                                   \
+    template hipError_t launch_state_in<R>(R*, long long, long long, long long, long long, const double*, hipStream_t);    \
+    template hipError_t launch_state_out<R>(const R*, long long, long long, long long, long long, R*, hipStream_t);
+NW_STATE_MOVE(float)
+NW_STATE_MOVE(double)
+#undef NW_STATE_MOVE
 
 hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t s) {
     const long long n4 = bytes / 16;

@@ -78,9 +78,11 @@ hipError_t launch_probe(const R* u, long long cs, long long ns, int nprobes, con
                         int n1, double* hist, int* slot, int cap, hipStream_t s, int nsteps = 1,
                         long long step_stride = 0, const int* stop = nullptr);
 hipError_t launch_zero_int(int* p, hipStream_t s);
-template <typename D, typename S>
-hipError_t launch_convert(D* dst, long long dcs, long long dns, const S* src, long long scs, long long sns, long long n,
-                          int ncomp, hipStream_t s);
+// Nodes p0 .. p0 + n - 1 of a device state from, to a host slot of six blocks of n values.
+template <typename R>
+hipError_t launch_state_in(R* u, long long cs, long long ns, long long p0, long long n, const double* slot, hipStream_t s);
+template <typename R>
+hipError_t launch_state_out(const R* u, long long cs, long long ns, long long p0, long long n, R* slot, hipStream_t s);
 hipError_t launch_copy(const void* src, void* dst, long long bytes, hipStream_t s);
 hipError_t launch_fill(double* p, long long n, double v, hipStream_t s);
 

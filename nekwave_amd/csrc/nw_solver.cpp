@@ -42,6 +42,10 @@ int upload_gll_tables(int device) {
 // LSRK45 coefficients, Carpenter & Kennedy (1994) (dg_solver.cpp:58-69).
 constexpr int kStages = 5;  // LSRK45 stages per step
 constexpr int kResidentSteps = 1024;        // steps of one resident launch, at most
+// Uploads of this many values take the runtime's copy (38 GB/s pageable; 12.6 MB 0.38
+// against 0.45 ms staged); smaller ones the staging slots (one launch and one wait:
+// 0.4 MB 31 against 113 us), larger ones too (100 MB 2.2 against 3.7 ms).
+constexpr size_t kPlainCopyFrom = (1u << 20) / 8, kPlainCopyTo = (32u << 20) / 8;
 constexpr long long kSnapBytes = 32 << 20;  // probed elements' fields kept per resident launch
 static const double kRkA[kStages] = {0.0, -567301805773.0 / 1357537059087.0,
                                      -2404267990393.0 / 2016746695238.0, -3550918686646.0 / 2091501179385.0,
@@ -213,7 +217,11 @@ void Solver::release() {
     drop_graphs();
     for (void* p : allocs) (void)hipFree(p);
     allocs.clear();
-    if (h_stop) (void)hipHostFree(h_stop);
+    if (h_page) {
+        (void)hipHostFree(h_page);
+        stage_release();
+    }
+    h_page = nullptr;
     h_stop = nullptr;
     release_resident();
     if (ev0) (void)hipEventDestroy(ev0);
@@ -341,7 +349,10 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
     const size_t ksz = (prec == kFP32 || prec == kBF16X3) ? 4 : 8;
     if ((st = dalloc(reinterpret_cast<void**>(&d_dt), 8))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_diag_part), sizeof(double) * 3 * diag_blocks()))) return st;
-    if ((st = dalloc(reinterpret_cast<void**>(&d_diag_out), sizeof(double) * 3))) return st;
+    NW_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_page), 128, hipHostMallocDefault));
+    stage_retain();
+    h_stop = reinterpret_cast<int*>(h_page + 8);
+    *h_stop = 0;
     long long max_inst = 0;
     for (const Instance& I : inst) max_inst = std::max(max_inst, I.npts);
     if ((st = dalloc(reinterpret_cast<void**>(&d_stage), sizeof(double) * 6 * max_inst))) return st;
@@ -549,20 +560,21 @@ int Solver::upload(int ix, const double* host, size_t n) {
     const Instance& I = inst[ix];
     NW_CHECK_ARG(host != nullptr && n == size_t(6 * I.npts), "upload: size must be 6*npts");
     NW_TRY_HIP(hipSetDevice(device));
-    const long long P = I.npts, S = stride;
-    if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(hipMemcpy2DAsync(d_state, S * 8, host, P * 8, P * 8, 6, hipMemcpyHostToDevice, stream));
+    int st;
+    if (device_pointer(host)) {
+        std::vector<double> h(n);
+        NW_TRY_HIP(hipMemcpy(h.data(), host, 8 * n, hipMemcpyDeviceToHost));
+        st = upload_state(device, stream, h.data(), I.npts, state_of(I));
+    } else if (n >= kPlainCopyFrom && n < kPlainCopyTo) {
+        NW_TRY_HIP(hipMemcpyAsync(d_stage, host, 8 * n, hipMemcpyHostToDevice, stream));
+        const DeviceState d = state_of(I);
+        if (d.f64) NW_TRY_HIP(launch_state_in(static_cast<double*>(d.data), d.cs, d.ns, 0, I.npts, d_stage, stream));
+        else NW_TRY_HIP(launch_state_in(static_cast<float*>(d.data), d.cs, d.ns, 0, I.npts, d_stage, stream));
+        st = NW_OK;
     } else {
-        // host blocks [Ex|..|Hz] -> node-major device layout (6 values per node)
-        NW_TRY_HIP(hipMemcpyAsync(d_stage, host, 8 * 6 * P, hipMemcpyHostToDevice, stream));
-        if (prec == kFP64) {
-            double* dst = static_cast<double*>(d_u[parity_of(I)]) + 6 * I.node_base;
-            NW_TRY_HIP((launch_convert<double, double>(dst, 1, 6, d_stage, P, 1, P, 6, stream)));
-        } else {
-            float* dst = static_cast<float*>(d_u[parity_of(I)]) + 6 * I.node_base;
-            NW_TRY_HIP((launch_convert<float, double>(dst, 1, 6, d_stage, P, 1, P, 6, stream)));
-        }
+        st = upload_state(device, stream, host, I.npts, state_of(I));
     }
+    if (st) return st;
     NW_TRY_HIP(hipStreamSynchronize(stream));
     uploaded = true;
     return NW_OK;
@@ -574,21 +586,22 @@ int Solver::download(int ix, double* host, size_t n) {
     const Instance& I = inst[ix];
     NW_CHECK_ARG(host != nullptr && n == size_t(6 * I.npts), "download: size must be 6*npts");
     NW_TRY_HIP(hipSetDevice(device));
-    const long long P = I.npts, S = stride;
-    if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(hipMemcpy2DAsync(host, P * 8, d_state, S * 8, P * 8, 6, hipMemcpyDeviceToHost, stream));
-    } else {
-        if (prec == kFP64) {
-            const double* src = static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base;
-            NW_TRY_HIP((launch_convert<double, double>(d_stage, P, 1, src, 1, 6, P, 6, stream)));
-        } else {
-            const float* src = static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base;
-            NW_TRY_HIP((launch_convert<double, float>(d_stage, P, 1, src, 1, 6, P, 6, stream)));
-        }
-        NW_TRY_HIP(hipMemcpyAsync(host, d_stage, 8 * 6 * P, hipMemcpyDeviceToHost, stream));
+    if (device_pointer(host)) {
+        std::vector<double> h(n);
+        const int st = download_state(device, stream, h.data(), I.npts, state_of(I));
+        if (st) return st;
+        NW_TRY_HIP(hipMemcpy(host, h.data(), 8 * n, hipMemcpyHostToDevice));
+        return NW_OK;
     }
-    NW_TRY_HIP(hipStreamSynchronize(stream));
-    return NW_OK;
+    return download_state(device, stream, host, I.npts, state_of(I));
+}
+
+// Where instance I's current state lies.
+DeviceState Solver::state_of(const Instance& I) const {
+    if (pipe == NW_PIPE_PLAIN) return {d_state, true, stride, 1};
+    char* u = static_cast<char*>(d_u[parity_of(I)]);
+    if (prec == kFP64) return {u + 48 * I.node_base, true, 1, 6};
+    return {u + 24 * I.node_base, false, 1, 6};
 }
 
 int Solver::set_dt(double dt) {
@@ -819,6 +832,7 @@ int Solver::set_probes(const Mesh& m, int n, const double* xyz, int capacity) {
     NW_TRY_HIP(hipStreamSynchronize(stream));
     nprobes = n;
     probe_cap = capacity;
+    probe_taken = 0;
     return NW_OK;
 }
 
@@ -831,6 +845,7 @@ int Solver::probe_sample() {
     int st = enqueue_probe(pipe == NW_PIPE_FUSED ? parity_of(inst[0]) : 0);
     if (st) return st;
     NW_TRY_HIP(hipStreamSynchronize(stream));
+    ++probe_taken;
     return NW_OK;
 }
 
@@ -842,20 +857,19 @@ int Solver::probe_history(double* host, int max_records, int* nrecords) {
     NW_CHECK_ARG(nrecords != nullptr, "null record count");
     if (nprobes <= 0) { *nrecords = 0; return NW_OK; }
     NW_TRY_HIP(hipSetDevice(device));
-    int taken = 0;
-    NW_TRY_HIP(hipMemcpyAsync(&taken, d_probe_slot, sizeof(int), hipMemcpyDeviceToHost, stream));
-    NW_TRY_HIP(hipStreamSynchronize(stream));
-    if (taken > probe_cap) {
+    if (probe_taken > probe_cap) {
         set_error("probe history overflow: fetch at least every capacity steps");
         return NW_ERR_STATE;
     }
+    const int taken = static_cast<int>(probe_taken);
     NW_CHECK_ARG(host != nullptr || taken == 0, "null host buffer");
     NW_CHECK_ARG(max_records >= taken, "host buffer holds fewer records than were taken");
-    if (taken > 0)
-        NW_TRY_HIP(hipMemcpyAsync(host, d_probe_hist, sizeof(double) * 6 * size_t(nprobes) * taken,
-                                  hipMemcpyDeviceToHost, stream));
-    NW_TRY_HIP(launch_zero_int(d_probe_slot, stream));
-    NW_TRY_HIP(hipStreamSynchronize(stream));
+    if (taken > 0) {
+        const int st = download_bytes(device, stream, host, d_probe_hist, sizeof(double) * 6 * size_t(nprobes) * taken);
+        if (st) return st;
+    }
+    NW_TRY_HIP(launch_zero_int(d_probe_slot, stream));  // before any later record, in stream order
+    probe_taken = 0;
     *nrecords = taken;
     return NW_OK;
 }
@@ -1065,6 +1079,7 @@ int Solver::launch_steps(double dt, int nsteps) {
     if (resident && (st = enqueue_resident(dt, nsteps))) return st;
     for (int x = 0; x < 2; ++x)
         if (!sets[x].segs.empty() && !(x == 1 && resident) && (st = enqueue_staged(sets[x], dt, nsteps))) return st;
+    if (nprobes > 0) probe_taken += nsteps;
     return NW_OK;
 }
 
@@ -1202,8 +1217,6 @@ int Solver::init_resident(const Mesh* const* meshes) {
     if ((st = dalloc(reinterpret_cast<void**>(&d_stop), sizeof(int)))) return st;
     NW_TRY_HIP(hipMemsetAsync(d_xchg, 0, size_t(bytes), stream));  // no tag matches an epoch that has not been stored
     NW_TRY_HIP(hipMemsetAsync(d_stop, 0, sizeof(int), stream));
-    NW_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_stop), sizeof(int), hipHostMallocDefault));
-    *h_stop = 0;
     return NW_OK;
 }
 
@@ -1301,18 +1314,17 @@ int Solver::diag(int ix, nw_diag* out) {
     const ElemMat* mat = I.media ? d_mat + I.elem_base : nullptr;
     const ElemGeom* geom = d_geom + I.elem_base;
     if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(launch_diag<double>(d_state, stride, 1, npts, n1, d_met[3], nullptr, mat, d_diag_part, d_diag_out,
+        NW_TRY_HIP(launch_diag<double>(d_state, stride, 1, npts, n1, d_met[3], nullptr, mat, d_diag_part, h_page,
                                        stream));
     } else if (prec == kFP64) {
         NW_TRY_HIP(launch_diag<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
-                                       nullptr, geom, mat, d_diag_part, d_diag_out, stream));
+                                       nullptr, geom, mat, d_diag_part, h_page, stream));
     } else {
         NW_TRY_HIP(launch_diag<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
-                                      nullptr, geom, mat, d_diag_part, d_diag_out, stream));
+                                      nullptr, geom, mat, d_diag_part, h_page, stream));
     }
-    double h[3];
-    NW_TRY_HIP(hipMemcpyAsync(h, d_diag_out, sizeof(h), hipMemcpyDeviceToHost, stream));
     NW_TRY_HIP(hipStreamSynchronize(stream));
+    const volatile double* h = h_page;
     out->energy = h[0];
     out->max_e = h[1];
     out->max_h = h[2];
@@ -1331,18 +1343,17 @@ int Solver::rel_l2(int ix, const double* ref, size_t n, double* out) {
     NW_TRY_HIP(hipMemcpyAsync(d_stage, ref, 8 * 6 * I.npts, hipMemcpyHostToDevice, stream));
     const ElemGeom* geom = d_geom + I.elem_base;
     if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(launch_l2<double>(d_state, stride, 1, d_stage, npts, n1, d_met[3], nullptr, d_diag_part, d_diag_out,
+        NW_TRY_HIP(launch_l2<double>(d_state, stride, 1, d_stage, npts, n1, d_met[3], nullptr, d_diag_part, h_page,
                                      stream));
     } else if (prec == kFP64) {
         NW_TRY_HIP(launch_l2<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts,
-                                     I.n1, nullptr, geom, d_diag_part, d_diag_out, stream));
+                                     I.n1, nullptr, geom, d_diag_part, h_page, stream));
     } else {
         NW_TRY_HIP(launch_l2<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts, I.n1,
-                                    nullptr, geom, d_diag_part, d_diag_out, stream));
+                                    nullptr, geom, d_diag_part, h_page, stream));
     }
-    double h[2];
-    NW_TRY_HIP(hipMemcpyAsync(h, d_diag_out, sizeof(h), hipMemcpyDeviceToHost, stream));
     NW_TRY_HIP(hipStreamSynchronize(stream));
+    const double h[2] = {static_cast<volatile double*>(h_page)[0], static_cast<volatile double*>(h_page)[1]};
     *out = h[1] > 0.0 ? std::sqrt(h[0] / h[1]) : (h[0] > 0.0 ? HUGE_VAL : 0.0);
     return NW_OK;
 }

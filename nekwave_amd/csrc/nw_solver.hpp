@@ -7,6 +7,7 @@
 #include "nw_fused.hpp"
 #include "nw_mesh.hpp"
 #include "nw_resident.hpp"
+#include "nw_transfer.hpp"
 
 namespace nw {
 
@@ -73,7 +74,9 @@ struct Solver {
     // shared
     double* d_dt = nullptr;
     double* d_diag_part = nullptr;
-    double* d_diag_out = nullptr;
+    // pinned host memory that kernels write: diagnostics (3 doubles), and from byte
+    // 64 on the number of a resident launch that gave up
+    double* h_page = nullptr;
     double* d_stage = nullptr;
     ElemMat* d_mat = nullptr;
     ElemGeom* d_geom = nullptr;
@@ -104,7 +107,7 @@ struct Solver {
     int4* d_rnbr = nullptr;
     unsigned long long* d_xchg = nullptr;
     int* d_stop = nullptr;
-    int* h_stop = nullptr;  // host memory the kernel writes
+    int* h_stop = nullptr;  // in h_page
     void* d_snap = nullptr;        // probed elements' fields after each step of a launch
     int* d_snap_slot = nullptr;    // per element: its slot in d_snap, -1 none
     long long* d_snap_base = nullptr;  // per probe: its element's offset in a step's record
@@ -118,6 +121,7 @@ struct Solver {
     // probes (device-side ProbeManager): per probe the node base of its element and
     // the 1-D Lagrange weights Lr, Ls, Lt; a history of `probe_cap` records
     int nprobes = 0, probe_cap = 0;
+    long long probe_taken = 0;  // records since the history was last fetched
     long long* d_probe_base = nullptr;
     double* d_probe_w = nullptr;
     double* d_probe_hist = nullptr;
@@ -144,6 +148,8 @@ struct Solver {
     // non-temporal k accesses of segment sg under a tile option: the tuned
     // choice, else the default rule (fused_stream_k)
     int stream_of(const Segment& sg, int option) const;
+
+    DeviceState state_of(const Instance& I) const;
 
    private:
     int dalloc(void** p, size_t bytes);
