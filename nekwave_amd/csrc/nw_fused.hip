@@ -131,11 +131,27 @@ void k_fused_stage(FusedArgs A) {
     // one element per workgroup) -- 1: FP32 products, 2: split BF16 products
     // (hi*hi + hi*lo + lo*hi with FP32 accumulation) -- else (0) on the vector ALUs.
     static_assert(!MX || (N1 == 8 && EPW == 1 && sizeof(R) == 4), "matrix-core volume shape");
-    __shared__ R sU[EPW][6][NP];
+    // QB (n1 = 8, FP32, vector-ALU volume): contractions by quad broadcast
+    // (line8x3); wave k holds plane k.  Planes are 72 words apart there, so that lines
+    // along t fall into different banks.  A line costs each lane two 4-byte LDS reads
+    // per field; with the lines copied for 16-byte reads it was eight values read and
+    // two more written per node and field (LDS active 70 -> 61 % of busy cycles,
+    // registers 124 -> 112): 20^3 jittered 79.5 -> 77.6 us per stage, 16^3 jittered 40.7
+    // both ways.
+    constexpr bool QB = N1 == 8 && EPW == 1 && sizeof(R) == 4 && !MX;
+    // QB on affine segments: a face point reads its minus side from sU (rows 9 words
+    // apart, so the nodes of every face fall into different banks) and its normal from
+    // the element record, and no face rows (sC) pass through LDS: with QB
+    // 16^3 39.7 -> 38.0 us per stage, 32^3 313.4 -> 309.1.  (With per-node geometry, evaluating the
+    // face point's row costs more than the rows: 16^3 jittered 41.2 -> 42.8.)
+    constexpr bool ROWS = !(QB && AFF);
+    constexpr int RS = ROWS ? N1 : 9, PL = QB ? 72 : N2;  // row and plane strides of sU
+    __shared__ R sU[EPW][6][PL * N1];
+    __shared__ R sT[QB ? 6 : 1][QB ? PL * N1 : 1];  // QB: t-derivatives, handed across waves
     __shared__ R sF[EPW * NF + 1][6];  // face terms dA*F; the last row stays zero
     constexpr int SPARE = sizeof(R) == 4 ? 64 : 0;  // spare face rows (branch-free writes, FP32)
-    __shared__ R sC[EPW * NF + SPARE][9];  // per face point: Nanson vector, minus-side trace (6)
-    __shared__ R sD[N2];               // D, row-major: sD[i * N1 + l] = D_il
+    __shared__ R sC[ROWS ? EPW * NF + SPARE : 1][9];  // per face point: Nanson vector, minus-side trace (6)
+    __shared__ __attribute__((aligned(16))) R sD[N2];  // D, row-major: sD[i * N1 + l] = D_il
     __shared__ ElemRec sE[2][EPW];     // element records, double-buffered over groups
     // FP32 fields: the records' 24 trilinear coefficients rounded to R once per
     // group (the per-node geometry reads them); FP64 fields read sE itself
@@ -144,12 +160,11 @@ void k_fused_stage(FusedArgs A) {
     // the i = n1-1 plane of the last slot of the previous group (its pre-stage
     // fields), rows of 7 words so a wave's reads of consecutive rows do not conflict
     __shared__ R sP3[N2][7];
-    // n1 = 8, 9, FP32, vector-ALU volume: the fields again with the s-lines
-    // (i, k) and t-lines (i, j) contiguous, lines 12 words apart (16-byte
-    // aligned; at n1 = 8 eight lines cover all 32 banks), so those directions
+    // n1 = 9, FP32: the fields again with the s-lines (i, k) and t-lines (i, j)
+    // contiguous, lines 12 words apart (16-byte aligned), so those directions
     // read their lines with 16-byte accesses instead of 4-byte ones at strides
-    // of n1 and n1^2 words (measured faster at n1 = 8, 9; slower at 6 and 7)
-    constexpr bool TL = (N1 == 8 || N1 == 9) && EPW == 1 && sizeof(R) == 4 && !MX;
+    // of n1 and n1^2 words (measured faster at n1 = 9; slower at 6 and 7)
+    constexpr bool TL = N1 == 9 && EPW == 1 && sizeof(R) == 4 && !MX;
     constexpr int RW = 12;
     __shared__ __attribute__((aligned(16))) R sUs[TL ? 6 : 1][TL ? RW * N2 : 1];
     __shared__ __attribute__((aligned(16))) R sUt[TL ? 6 : 1][TL ? RW * N2 : 1];
@@ -176,6 +191,7 @@ void k_fused_stage(FusedArgs A) {
     const int es = tid / NP;
     const int m = tid - es * NP;
     const int i = m % N1, j = (m / N1) % N1, k = m / N2;
+    const int um = i + RS * j + PL * k;  // the node's place in sU
     // FP32 at n1 = 8, one element per workgroup: each wave holds one k-plane, so
     // whether its nodes lie on a t-face is wave-uniform and the t-face row
     // writes and t-lift reads of the six interior planes are skipped by a
@@ -318,7 +334,7 @@ void k_fused_stage(FusedArgs A) {
             // at n1 = 8 with one element per workgroup a wave holds one face: uniform
             if constexpr (SF) kind = __builtin_amdgcn_readfirstlane(kind);
             P.kind[t] = kind;
-            const unsigned idx = (kind == kGather && fp < EPW * NF) ? unsigned(b.x + p * b.y + q * b.z) : nd;
+            const unsigned idx = (kind == kGather && fp < EPW * NF) ? unsigned(b.x + __mul24(p, b.y) + __mul24(q, b.z)) : nd;
             ld6(rU, idx * UB, P.up[t]);
         }
     };
@@ -368,6 +384,12 @@ void k_fused_stage(FusedArgs A) {
     };
     R geo[10];
     geometry(0, geo);
+
+    // !ROWS: the place in sU of this thread's face point (of face wface)
+    const int fpp = (tid & 63) % N1, fqq = (tid & 63) / N1;
+    const int fnode = (wface == 1 || wface == 3) ? (wface == 1 ? N1 - 1 : 0) + RS * fpp + PL * fqq
+                      : (wface < 3)              ? fpp + RS * (wface == 2 ? N1 - 1 : 0) + PL * fqq
+                                                 : fpp + RS * fqq + PL * (wface == 5 ? N1 - 1 : 0);
 
     for (int t = 0; t <= tl; ++t) {
         const int g = gA;
@@ -427,7 +449,9 @@ void k_fused_stage(FusedArgs A) {
 #pragma unroll
             for (int c2 = 0; c2 < 6; ++c2) o[3 + c2] = cur.u[c2];
         };
-        if constexpr (SPARE > 0) {
+        if constexpr (!ROWS) {
+            // the face points read sU
+        } else if constexpr (SPARE > 0) {
             const int spare = EPW * NF + (tid & 63);
             const int rs = j == 0 ? es * NF + 0 * N2 + i + N1 * k : (j == N1 - 1 ? es * NF + 2 * N2 + i + N1 * k : spare);
             const int rr = i == N1 - 1 ? es * NF + 1 * N2 + j + N1 * k : (i == 0 ? es * NF + 3 * N2 + j + N1 * k : spare);
@@ -446,7 +470,7 @@ void k_fused_stage(FusedArgs A) {
             if (k == N1 - 1) row(b + 5 * N2 + i + N1 * j, Ctx, Cty, Ctz);
         }
 #pragma unroll
-        for (int c = 0; c < 6; ++c) sU[es][c][m] = cur.u[c];
+        for (int c = 0; c < 6; ++c) sU[es][c][um] = cur.u[c];
         if constexpr (TL) {
 #pragma unroll
             for (int c = 0; c < 6; ++c) {
@@ -466,6 +490,17 @@ void k_fused_stage(FusedArgs A) {
         // ---- 2. volume: reference derivatives (local_grad3, dg_kernels.cu:101-124)
         // folded straight into J * curl (dg_kernels.cu:140-149) ----
         R cE[3] = {R(0), R(0), R(0)}, cH[3] = {R(0), R(0), R(0)};
+        // a[3]: derivatives of E (h = 0) or H along d.  J d/dx_e of component c gets
+        // a * C_d,e; curl u = (dy u_z - dz u_y, dz u_x - dx u_z, dx u_y - dy u_x)
+        auto fold = [&](int d, int h, const R(&a)[3]) {
+            const R Cx = d == 0 ? Crx : (d == 1 ? Csx : Ctx);
+            const R Cy = d == 0 ? Cry : (d == 1 ? Csy : Cty);
+            const R Cz = d == 0 ? Crz : (d == 1 ? Csz : Ctz);
+            R* cv = h == 0 ? cE : cH;
+            cv[1] += a[0] * Cz; cv[2] -= a[0] * Cy;
+            cv[0] -= a[1] * Cz; cv[2] += a[1] * Cx;
+            cv[0] += a[2] * Cy; cv[1] -= a[2] * Cx;
+        };
         if constexpr (MX) {
             // 36 tasks (direction d, field c, half of the 64 lines), in pairs:
             // one v_mfma_f32_4x4x1_16b per column q of D and task.  Lane 4b + x
@@ -535,6 +570,43 @@ void k_fused_stage(FusedArgs A) {
                     for (int r = 0; r < 4; ++r) { sAt[c][9 * l0 + 4 * h + r] = a0[r]; sAt[c][9 * l1 + 4 * h + r] = a1[r]; }
                 }
             }
+        } else if constexpr (QB) {
+            float Dq[8];  // the lane's row of D, the same in every direction
+            int dr = i * N1;
+            pin(dr);  // read here, not kept in registers over the loop
+#pragma unroll
+            for (int q = 0; q < 8; ++q) Dq[q] = sD[dr + q];
+            // lane = (line, position): r lines (j, k), s lines (i, k) -- both in the
+            // wave's own plane -- and t lines (i, j = wave) across the planes
+            const int lr = (i & 3) + RS * j + PL * k, ls = j + RS * (i & 3) + PL * k, lt = j + RS * k + PL * (i & 3);
+            auto lines = [&](int h, int lo, int hi, R(&a)[3]) {
+                const R l[3] = {sU[0][3 * h][lo], sU[0][3 * h + 1][lo], sU[0][3 * h + 2][lo]};
+                const R u[3] = {sU[0][3 * h][hi], sU[0][3 * h + 1][hi], sU[0][3 * h + 2][hi]};
+                line8x3(Dq, l, u, a);
+            };
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                R a[3];
+                lines(h, lr, lr + 4, a);
+                fold(0, h, a);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                R a[3];
+                lines(h, ls, ls + 4 * RS, a);
+#pragma unroll
+                for (int c = 0; c < 3; ++c)  // lane (position j, line i) -> the node's lane (i, j)
+                    a[c] = __builtin_bit_cast(R, __builtin_amdgcn_ds_bpermute(4 * (j + 8 * i), __builtin_bit_cast(int, a[c])));
+                fold(1, h, a);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                R a[3];
+                lines(h, lt, lt + 4 * PL, a);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) sT[3 * h + c][j + RS * k + PL * i] = a[c];
+            }
+            pin(cE[0]); pin(cE[1]); pin(cE[2]); pin(cH[0]); pin(cH[1]); pin(cH[2]);
         } else {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {  // reference direction r, s, t: one row of D live at a time
@@ -542,9 +614,6 @@ void k_fused_stage(FusedArgs A) {
             R Dr[N1];
 #pragma unroll
             for (int q = 0; q < N1; ++q) Dr[q] = sD[row * N1 + q];
-            const R Cx = d == 0 ? Crx : (d == 1 ? Csx : Ctx);
-            const R Cy = d == 0 ? Cry : (d == 1 ? Csy : Cty);
-            const R Cz = d == 0 ? Crz : (d == 1 ? Csz : Ctz);
             // E then H: three fields' contractions as independent chains, interleaved
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -559,12 +628,7 @@ void k_fused_stage(FusedArgs A) {
                         a[c] += Dr[q] * v;
                     }
                 }
-                // J d/dx_e of component c gets a * C_d,e;
-                // curl u = (dy u_z - dz u_y, dz u_x - dx u_z, dx u_y - dy u_x)
-                R* cv = h == 0 ? cE : cH;
-                cv[1] += a[0] * Cz; cv[2] -= a[0] * Cy;
-                cv[0] -= a[1] * Cz; cv[2] += a[1] * Cx;
-                cv[0] += a[2] * Cy; cv[1] -= a[2] * Cx;
+                fold(d, h, a);
             }
             // keep each direction's contraction here: sinking it into the update
             // below would hold the fields' LDS values in registers
@@ -579,7 +643,21 @@ void k_fused_stage(FusedArgs A) {
             if (fp < EPW * NF) {
                 const int efs = fp / NF, r = fp - efs * NF;
                 const int f = r / N2, pq = r - f * N2, p = pq % N1, q = pq / N1;
-                const R* mine = &sC[fp][3];
+                R mine[6], N[3];  // minus-side trace, outward Nanson vector
+                if constexpr (!ROWS) {
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) mine[c] = sU[0][c][fnode];
+                    // outward: +-(cofactor row of the face's direction)
+                    const int dir = (wface == 1 || wface == 3) ? 0 : (wface < 3 ? 1 : 2);
+                    const R sg = (wface == 1 || wface == 2 || wface == 5) ? R(1) : R(-1);
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) N[c] = sg * R((&ER.g.c[0][0])[3 * dir + c]);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 6; ++c) mine[c] = sC[fp][3 + c];
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) N[c] = sC[fp][c];
+                }
                 R jE[3], jH[3];
                 const int kind = cur.kind[t];
                 if (kind == kMirror) {  // PEC mirror: [[E]] = -2 E-, [[H]] = 0 (dg_kernels.cu:244-251)
@@ -613,7 +691,7 @@ void k_fused_stage(FusedArgs A) {
                     }
                 }
                 // unit normal and area element (mesh.cpp:1032-1038)
-                const R Nx = sC[fp][0], Ny = sC[fp][1], Nz = sC[fp][2];
+                const R Nx = N[0], Ny = N[1], Nz = N[2];
                 R Ln, il;
                 norm_and_inverse(Nx * Nx + Ny * Ny + Nz * Nz, Ln, il);
                 const R nx = Nx * il, ny = Ny * il, nz = Nz * il;
@@ -638,20 +716,22 @@ void k_fused_stage(FusedArgs A) {
         if constexpr (MX) {  // fold the node's 18 derivatives into J * curl
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                const R Cx = d == 0 ? Crx : (d == 1 ? Csx : Ctx);
-                const R Cy = d == 0 ? Cry : (d == 1 ? Csy : Cty);
-                const R Cz = d == 0 ? Crz : (d == 1 ? Csz : Ctz);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     R a[3];
 #pragma unroll
                     for (int c = 0; c < 3; ++c)
                         a[c] = d == 0 ? sA[0][3 * h + c][m] : (d == 1 ? sA[1][3 * h + c][j + 8 * i + 64 * k] : sAt[3 * h + c][k + 9 * (i + 8 * j)]);
-                    R* cv = h == 0 ? cE : cH;
-                    cv[1] += a[0] * Cz; cv[2] -= a[0] * Cy;
-                    cv[0] -= a[1] * Cz; cv[2] += a[1] * Cx;
-                    cv[0] += a[2] * Cy; cv[1] -= a[2] * Cx;
+                    fold(d, h, a);
                 }
+            }
+        }
+
+        if constexpr (QB) {  // the t-derivatives, complete since the barrier
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const R a[3] = {sT[3 * h][um], sT[3 * h + 1][um], sT[3 * h + 2][um]};
+                fold(2, h, a);
             }
         }
 
@@ -701,7 +781,7 @@ void k_fused_stage(FusedArgs A) {
             for (int c = 0; c < 6; ++c) {
                 const R rhs = c < 3 ? sE_ * (cH[c] + LE[c] * Winv) : sH_ * (-cE[c - 3] + LH[c - 3] * Winv);
                 kn[c] = FIRST ? KR(dt) * KR(rhs) : KR(A.a) * kold[c] + KR(dt) * KR(rhs);
-                un[c] = R(KR(sU[es][c][m]) + KR(A.b) * kn[c]);
+                un[c] = R(KR(sU[es][c][um]) + KR(A.b) * kn[c]);
             }
             // written through L2 (whole lines): the kernel boundary, which writes
             // every dirty L2 line back for the other XCDs, has k's lines off its list.

@@ -57,12 +57,13 @@ void k_resident(ResidentArgs A) {
     constexpr int FPT = (NF + NT - 1) / NT;     // face points per thread
     constexpr int PC = 6 * int(sizeof(R)) / 4;  // packets per face point
     constexpr int GW = AFF ? 10 : 24;           // geometry words per element
-    // QB: contractions by quad broadcast (line8x3); wave k holds plane k.  Planes are
-    // 72 words apart there, so lines along t fall into different banks.  A third less
+    // QB: contractions by quad broadcast (line8x3); wave k holds plane k.  Rows are 9
+    // and planes 72 words apart there, so that lines in every direction and the nodes
+    // of every face fall into different banks.  A third less
     // LDS time (n1 = 8, 512 elements: 423 -> 285 LDS cycles per wave and stage), 4.6 ->
     // 4.2 us per stage; 1728 uniform elements 17.0 -> 15.6.
     constexpr bool QB = N1 == 8 && sizeof(R) == 4;
-    constexpr int PL = QB ? 72 : N2;
+    constexpr int RS = QB ? 9 : N1, PL = QB ? 72 : N2;  // row and plane strides of sU
     __shared__ R sU[EM][6][PL * N1];
     __shared__ R sT[QB ? 6 : 1][QB ? PL * N1 : 1];  // QB: t-derivatives, handed across waves
     __shared__ R sF[NF + 1][6];  // face terms dA*F; the last row stays zero
@@ -74,7 +75,7 @@ void k_resident(ResidentArgs A) {
 
     const int tid = threadIdx.x, m = tid;
     const int i = m % N1, j = (m / N1) % N1, k = m / N2;
-    const int at = i + N1 * j + PL * k;  // the node's place in sU
+    const int at = i + RS * j + PL * k;  // the node's place in sU
     const int el0 = A.elem0 + static_cast<int>(blockIdx.x) * A.per;  // first element of this workgroup
     const int cnt = min(A.per, A.elem0 + A.nelt - el0);
     const R* uin = static_cast<const R*>(A.uin);
@@ -112,7 +113,7 @@ void k_resident(ResidentArgs A) {
         fpq[t] = pq;
         own[t] = 8u * (unsigned((el0 - A.elem0) * 6 + f) * (PC * N2) + unsigned(pq));
         const int ln = face_local_node<N1>(f, p, q);
-        fnode[t] = ln + (PL - N2) * (ln / N2);
+        fnode[t] = ln % N1 + RS * (ln / N1 % N1) + PL * (ln / N2);
         wpq[t] = R(c_gll.w[N1][p] * c_gll.w[N1][q]);
     }
     __syncthreads();
@@ -218,7 +219,7 @@ void k_resident(ResidentArgs A) {
                 // nine tangents and three rows)
                 int ln = fnode[t];
                 if constexpr (!KEEP) pin(ln);
-                const R r = sZ[ln % N1], q = sZ[(ln % PL) / N1], w = sZ[ln / PL];
+                const R r = sZ[ln % PL % RS], q = sZ[ln % PL / RS], w = sZ[ln / PL];
                 R T[2][3];
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
@@ -341,7 +342,7 @@ void k_resident(ResidentArgs A) {
                     // lane = (line, position): r lines (j, k), s lines (i, k) -- both in the
                     // wave's own plane -- and t lines (i, j = wave) across the planes
                     if constexpr (!KEEP) row_of_D();
-                    const int lr = (i & 3) + N1 * j + PL * k, ls = j + N1 * (i & 3) + PL * k, lt = j + N1 * k + PL * (i & 3);
+                    const int lr = (i & 3) + RS * j + PL * k, ls = j + RS * (i & 3) + PL * k, lt = j + RS * k + PL * (i & 3);
                     auto lines = [&](int h, int lo, int hi, R (&a)[3]) {
                         const R l[3] = {sU[x][3 * h][lo], sU[x][3 * h + 1][lo], sU[x][3 * h + 2][lo]};
                         const R u[3] = {sU[x][3 * h][hi], sU[x][3 * h + 1][hi], sU[x][3 * h + 2][hi]};
@@ -356,7 +357,7 @@ void k_resident(ResidentArgs A) {
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         R a[3];
-                        lines(h, ls, ls + 4 * N1, a);
+                        lines(h, ls, ls + 4 * RS, a);
 #pragma unroll
                         for (int c = 0; c < 3; ++c)  // lane (position j, line i) -> the node's lane (i, j)
                             a[c] = __builtin_bit_cast(R, __builtin_amdgcn_ds_bpermute(4 * (j + 8 * i), __builtin_bit_cast(int, a[c])));
@@ -368,7 +369,7 @@ void k_resident(ResidentArgs A) {
                         R a[3];
                         lines(h, lt, lt + 4 * PL, a);
 #pragma unroll
-                        for (int c = 0; c < 3; ++c) sT[3 * h + c][j + N1 * k + PL * i] = a[c];
+                        for (int c = 0; c < 3; ++c) sT[3 * h + c][j + RS * k + PL * i] = a[c];
                     }
                     pin(cE[0]); pin(cE[1]); pin(cE[2]); pin(cH[0]); pin(cH[1]); pin(cH[2]);
                 } else {
