@@ -13,7 +13,7 @@ Prints one JSON line: DOF-updates/s of the FP32 fused path (value: the median
 of five back-to-back timings of exactly K steps, after an untimed clock-settling
 run and W warm-up steps), the roofline of the fused stage kernel (algorithmic
 bytes per launch / mean launch time from HIP events on the solver's stream), the
-FP64 fused and FP64 reference-decomposed ("plain") rates, FP32 fields with FP64
+FP64 fused and FP64 stored-geometry ("plain") rates, FP32 fields with FP64
 LSRK registers, the FP32 relative L2 error against the FP64 path after 1000 steps
 with the energy drift of both, the PEC-cube TM110 case (relative L2 to the
 analytic mode, energy drift), the Case loop with on-device probes against the

@@ -241,7 +241,8 @@ class Mesh:
 
 class DgSolver:
     """Reference DgSolver.  Extensions: precision ('fp64', 'fp32', 'fp32_k64'),
-    pipeline ('fused' or 'plain' = the reference's 7-kernel stage), graphs, the
+    pipeline ('fused', or 'plain' = FP64 from the reference's per-node and
+    per-face-point arrays, any n1 in [2, 10]), graphs, the
     fused tile option (-1: tuned) and groups_per_cu, a cap on the fused launch's
     workgroups per CU (0: as many as fit)."""
 

@@ -19,7 +19,8 @@ BUILD = os.path.join(ROOT, "_build", "nekwave_amd")
 LIB = os.path.join(HERE, "libnekwave_amd.so")
 ARCH = os.environ.get("NW_OFFLOAD_ARCH", "gfx950")
 
-DEVICE_SOURCES = ["nw_fused.hip", "nw_resident_f64.hip", "nw_resident_f32.hip", "nw_resident_f32k64.hip", "nw_plain.hip"]
+DEVICE_SOURCES = ["nw_fused.hip", "nw_resident_f64.hip", "nw_resident_f32.hip", "nw_resident_f32k64.hip", "nw_plain.hip",
+                  "nw_plain_stage.hip"]
 HOST_SOURCES = ["nw_mesh.cpp", "nw_meshio.cpp", "nw_fields.cpp", "nw_resident.cpp", "nw_transfer.cpp", "nw_solver.cpp", "nw_api.cpp"]
 
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wno-unused-result",

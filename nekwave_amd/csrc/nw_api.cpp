@@ -446,7 +446,7 @@ NW_API int nw_launch_inv_mass(double* rhs, const double* jac, const double* w3, 
 NW_API int nw_launch_lsrk45_update(double* st, double* k, const double* rhs, double a, double b, double dt,
                                    int64_t npts, int64_t S, void* stream) {
     NW_CHECK_ARG(S >= npts, "lsrk: stride < npts");
-    NW_TRY_HIP(nw::launch_lsrk(st, k, rhs, a, b, nullptr, dt, npts, S, hs(stream)));
+    NW_TRY_HIP(nw::launch_lsrk(st, k, rhs, a, b, dt, npts, S, hs(stream)));
     return NW_OK;
 }
 NW_API int nw_launch_pack_halo(const double* st, double* buf, const int* vol, const int* off, const int* sizes,

@@ -16,6 +16,7 @@
 #include "nw_plain.hpp"
 
 #include "nw_fused.hpp"
+#include "nw_plain_device.hpp"
 
 namespace nw {
 namespace {
@@ -74,15 +75,9 @@ __global__ __launch_bounds__(EPW* N1* N1) void k_volume_curl(
         }
         const long long p = nb + N2 * k;
         const double w = w3g[l + N2 * k] * jac[p];
-        const double u1rw = a1r * w, u1sw = a1s * w, u1tw = a1t * w;
-        const double u2rw = a2r * w, u2sw = a2s * w, u2tw = a2t * w;
-        const double u3rw = a3r * w, u3sw = a3s * w, u3tw = a3t * w;
-        const double Rx = rx[p], Sx = sx[p], Tx = tx[p], Ry = ry[p], Sy = sy[p], Ty = ty[p];
-        const double Rz = rz[p], Sz = sz[p], Tz = tz[p];
-        const double o1 = (u3rw * Ry + u3sw * Sy + u3tw * Ty) - (u2rw * Rz + u2sw * Sz + u2tw * Tz);
-        const double o2 = (u1rw * Rz + u1sw * Sz + u1tw * Tz) - (u3rw * Rx + u3sw * Sx + u3tw * Tx);
-        const double o3 = (u2rw * Rx + u2sw * Sx + u2tw * Tx) - (u1rw * Ry + u1sw * Sy + u1tw * Ty);
-        w1[p] = sign * o1; w2[p] = sign * o2; w3o[p] = sign * o3;
+        const double met[9] = {rx[p], sx[p], tx[p], ry[p], sy[p], ty[p], rz[p], sz[p], tz[p]};
+        const Vec3 o = plain_curl({a1r, a2r, a3r}, {a1s, a2s, a3s}, {a1t, a2t, a3t}, w, met);
+        w1[p] = sign * o.x; w2[p] = sign * o.y; w3o[p] = sign * o.z;
     }
 }
 
@@ -116,37 +111,25 @@ __global__ void k_flux(const double* __restrict__ st, const double* __restrict__
                        double c0, long long tfp, long long S, const int* __restrict__ vM, const double* __restrict__ eps,
                        const double* __restrict__ mu, const int* __restrict__ ghost_elem, int np, long long npts) {
     for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
-        const double Exm = fEN[p], Eym = fEN[tfp + p], Ezm = fEN[2 * tfp + p];
-        const double Hxm = fHN[p], Hym = fHN[tfp + p], Hzm = fHN[2 * tfp + p];
+        const Vec3 Em = {fEN[p], fEN[tfp + p], fEN[2 * tfp + p]}, Hm = {fHN[p], fHN[tfp + p], fHN[2 * tfp + p]};
         const int v = vP[p];
         const bool mirror = bc[p] != 0 || v < 0;
-        double dEx, dEy, dEz, dHx, dHy, dHz;
+        Vec3 dE, dH, fH, fE;
         if (mirror) {
-            dEx = -2.0 * Exm; dEy = -2.0 * Eym; dEz = -2.0 * Ezm; dHx = 0.0; dHy = 0.0; dHz = 0.0;
+            dE = {-2.0 * Em.x, -2.0 * Em.y, -2.0 * Em.z};
+            dH = {0.0, 0.0, 0.0};
         } else {
-            dEx = st[v] - Exm; dEy = st[S + v] - Eym; dEz = st[2 * S + v] - Ezm;
-            dHx = st[3 * S + v] - Hxm; dHy = st[4 * S + v] - Hym; dHz = st[5 * S + v] - Hzm;
+            dE = {st[v] - Em.x, st[S + v] - Em.y, st[2 * S + v] - Em.z};
+            dH = {st[3 * S + v] - Hm.x, st[4 * S + v] - Hm.y, st[5 * S + v] - Hm.z};
         }
-        const double n_x = nxa[p], n_y = nya[p], n_z = nza[p];
-        const double nxEx = n_y * dEz - n_z * dEy, nxEy = n_z * dEx - n_x * dEz, nxEz = n_x * dEy - n_y * dEx;
-        const double nxHx = n_y * dHz - n_z * dHy, nxHy = n_z * dHx - n_x * dHz, nxHz = n_x * dHy - n_y * dHx;
-        const double nnEx = n_y * nxEz - n_z * nxEy, nnEy = n_z * nxEx - n_x * nxEz, nnEz = n_x * nxEy - n_y * nxEx;
-        const double nnHx = n_y * nxHz - n_z * nxHy, nnHy = n_z * nxHx - n_x * nxHz, nnHz = n_x * nxHy - n_y * nxHx;
-        double fHx, fHy, fHz, fEx, fEy, fEz;
-        if (!eps) {
-            fHx = -0.5 * nxEx - 0.5 * c0 * nnHx; fHy = -0.5 * nxEy - 0.5 * c0 * nnHy; fHz = -0.5 * nxEz - 0.5 * c0 * nnHz;
-            fEx = 0.5 * nxHx - 0.5 * c0 * nnEx; fEy = 0.5 * nxHy - 0.5 * c0 * nnEy; fEz = 0.5 * nxHz - 0.5 * c0 * nnEz;
-        } else {
-            const int em = vM[p] / np;
-            const int ep = mirror ? em : (v < npts ? v / np : ghost_elem[v - npts]);
-            const double Zm = sqrt(mu[em] / eps[em]), Zp = sqrt(mu[ep] / eps[ep]);
-            const double Ym = 1.0 / Zm, Yp = 1.0 / Zp;
-            const double iz = 1.0 / (Zp + Zm), iy = 1.0 / (Yp + Ym);
-            fHx = (-Yp * nxEx - c0 * nnHx) * iy; fHy = (-Yp * nxEy - c0 * nnHy) * iy; fHz = (-Yp * nxEz - c0 * nnHz) * iy;
-            fEx = (Zp * nxHx - c0 * nnEx) * iz; fEy = (Zp * nxHy - c0 * nnEy) * iz; fEz = (Zp * nxHz - c0 * nnEz) * iz;
+        int em = 0, ep = 0;
+        if (eps) {
+            em = vM[p] / np;
+            ep = mirror ? em : (v < npts ? v / np : ghost_elem[v - npts]);
         }
-        flux[p] = fHx; flux[tfp + p] = fHy; flux[2 * tfp + p] = fHz;
-        flux[3 * tfp + p] = fEx; flux[4 * tfp + p] = fEy; flux[5 * tfp + p] = fEz;
+        plain_flux(dE, dH, {nxa[p], nya[p], nza[p]}, c0, eps, mu, em, ep, fH, fE);
+        flux[p] = fH.x; flux[tfp + p] = fH.y; flux[2 * tfp + p] = fH.z;
+        flux[3 * tfp + p] = fE.x; flux[4 * tfp + p] = fE.y; flux[5 * tfp + p] = fE.z;
     }
 }
 
@@ -226,8 +209,7 @@ __global__ void k_inv_mass(double* __restrict__ rhs, const double* __restrict__ 
 }
 
 __global__ void k_lsrk(double* __restrict__ st, double* __restrict__ k, const double* __restrict__ rhs, double a,
-                       double b, const double* __restrict__ dtp, double dtv, long long npts, long long S) {
-    const double dt = dtp ? *dtp : dtv;
+                       double b, double dt, long long npts, long long S) {
     const long long n = 6 * npts;
     for (long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x < n; x += (long long)gridDim.x * blockDim.x) {
         const long long c = x / npts, p = x - c * npts;
@@ -301,8 +283,8 @@ __global__ void k_face_data(const int* __restrict__ fcode, const int* __restrict
                             long long npts, const double* __restrict__ jac, const double* __restrict__ rx,
                             const double* __restrict__ sx, const double* __restrict__ tx, const double* __restrict__ ry,
                             const double* __restrict__ sy, const double* __restrict__ ty, const double* __restrict__ rz,
-                            const double* __restrict__ sz, const double* __restrict__ tz, int* __restrict__ vM,
-                            int* __restrict__ vP, int* __restrict__ bc, double* __restrict__ nx, double* __restrict__ ny,
+                            const double* __restrict__ sz, const double* __restrict__ tz, int* __restrict__ vP,
+                            int* __restrict__ bc, double* __restrict__ nx, double* __restrict__ ny,
                             double* __restrict__ nz, double* __restrict__ dA) {
     const int n2 = n1 * n1, np = n2 * n1;
     for (long long P = blockIdx.x * (long long)blockDim.x + threadIdx.x; P < tfp; P += (long long)gridDim.x * blockDim.x) {
@@ -312,7 +294,6 @@ __global__ void k_face_data(const int* __restrict__ fcode, const int* __restrict
         int i, j, k;
         face_ijk(f, n1, p, q, i, j, k);
         const long long v = (long long)e * np + i + n1 * (j + n1 * k);
-        vM[P] = static_cast<int>(v);
         const double J = jac[v], w2 = c_gll.w[n1][p] * c_gll.w[n1][q];
         double Nx, Ny, Nz;
         switch (f) {
@@ -678,14 +659,6 @@ hipError_t launch_flux(const double* st, const double* fEN, const double* fHN, c
     return hipGetLastError();
 }
 
-hipError_t launch_lift(const double* flux, const double* dA, double* rhs, long long tfp, long long npts, int n1,
-                       hipStream_t s) {
-    if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_lift, dim3(grid_for(npts)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, n1,
-                       static_cast<const int*>(nullptr));
-    return hipGetLastError();
-}
-
 hipError_t launch_add_flux(const double* flux, const int* vM, const double* dA, double* rhs, long long tfp,
                            long long npts, hipStream_t s) {
     if (tfp <= 0) return hipSuccess;
@@ -713,10 +686,10 @@ hipError_t launch_inv_mass(double* rhs, const double* jac, const double* w3, int
     return hipGetLastError();
 }
 
-hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, const double* dtp, double dt,
+hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, double dt,
                        long long npts, long long S, hipStream_t s) {
     if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_lsrk, dim3(grid_for(6 * npts)), dim3(kBlock), 0, s, st, k, rhs, a, b, dtp, dt, npts, S);
+    hipLaunchKernelGGL(k_lsrk, dim3(grid_for(6 * npts)), dim3(kBlock), 0, s, st, k, rhs, a, b, dt, npts, S);
     return hipGetLastError();
 }
 
@@ -752,11 +725,11 @@ hipError_t launch_metrics(const double* corners, int n1, long long npts, double*
 }
 
 hipError_t launch_face_data(const int* fcode, const int* fbc, int n1, long long tfp, long long npts,
-                            const double* const* met10, int* vM, int* vP, int* bc, double* nx, double* ny, double* nz,
+                            const double* const* met10, int* vP, int* bc, double* nx, double* ny, double* nz,
                             double* dA, hipStream_t s) {
     if (tfp <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_face_data, dim3(grid_for(tfp)), dim3(kBlock), 0, s, fcode, fbc, n1, tfp, npts, met10[0],
-                       met10[1], met10[2], met10[3], met10[4], met10[5], met10[6], met10[7], met10[8], met10[9], vM, vP,
+                       met10[1], met10[2], met10[3], met10[4], met10[5], met10[6], met10[7], met10[8], met10[9], vP,
                        bc, nx, ny, nz, dA);
     return hipGetLastError();
 }

@@ -1,5 +1,6 @@
-// nw_plain.hpp -- launchers of the reference-decomposed FP64 kernels and the
-// device-side helpers (geometry setup, diagnostics, conversion, halo).
+// nw_plain.hpp -- launchers of the reference-decomposed FP64 kernels, the plain
+// pipeline's stage and the device-side helpers (geometry setup, diagnostics,
+// conversion, halo).
 #pragma once
 
 #include "nw_internal.hpp"
@@ -15,6 +16,23 @@ struct PlainVolumeArgs {
     int n1, nelt;
 };
 
+// One LSRK stage uin -> uout (node-major: component c of node p at 6 p + c; ghosts past
+// npts), k in component blocks of npts; face points in the element-major layout.
+struct PlainStageArgs {
+    const double* uin;
+    double *uout, *k;
+    const double *D, *w3;
+    const double* met[10];  // jac rx sx tx ry sy ty rz sz tz
+    const int *vP, *bc;
+    const double *nx, *ny, *nz, *dA;
+    const double *eps, *mu;  // per element, or null
+    const int* ghost_elem;
+    const double* dt;
+    double a, b, c0;
+    int nelt, npts;
+};
+hipError_t launch_plain_stage(int n1, const PlainStageArgs& a, hipStream_t s);
+
 int plain_upload_tables(const GllTables& t);
 
 hipError_t launch_volume_curl(const PlainVolumeArgs& a, hipStream_t s);
@@ -24,8 +42,6 @@ hipError_t launch_flux(const double* st, const double* fEN, const double* fHN, c
                        const double* nx, const double* ny, const double* nz, double* flux, double c0, long long tfp,
                        long long S, const int* vM, const double* eps, const double* mu, const int* ghost_elem, int np,
                        long long npts, hipStream_t s);
-hipError_t launch_lift(const double* flux, const double* dA, double* rhs, long long tfp, long long npts, int n1,
-                       hipStream_t s);
 // launch_add_flux with the reference's arguments (dg_kernels.hpp:46-50): nodes of
 // the element-major face layout gather their points in face order
 // (deterministic); points whose volIdxMinus departs from that layout are added
@@ -34,7 +50,7 @@ hipError_t launch_add_flux(const double* flux, const int* vM, const double* dA, 
                            long long npts, hipStream_t s);
 hipError_t launch_inv_mass(double* rhs, const double* jac, const double* w3, int nxyz, long long npts,
                            const double* eps, const double* mu, hipStream_t s);
-hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, const double* dtp, double dt,
+hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, double dt,
                        long long npts, long long S, hipStream_t s);
 // State layouts: component c of node p at c * cs + p * ns (the reference's
 // blocks [Ex|..|Hz]: cs = stride, ns = 1; node-major: cs = 1, ns = 6).
@@ -46,7 +62,7 @@ hipError_t launch_unpack(const R* buf, R* st, const int* off, const int* sizes, 
                          long long ns, hipStream_t s);
 hipError_t launch_metrics(const double* corners, int n1, long long npts, double* const* out13, hipStream_t s);
 hipError_t launch_face_data(const int* fcode, const int* fbc, int n1, long long tfp, long long npts,
-                            const double* const* met10, int* vM, int* vP, int* bc, double* nx, double* ny, double* nz,
+                            const double* const* met10, int* vP, int* bc, double* nx, double* ny, double* nz,
                             double* dA, hipStream_t s);
 int diag_blocks();
 template <typename R>

@@ -403,12 +403,14 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
         if ((st = dalloc(&d_recvbuf, rsz * 6 * nh))) return st;
     }
 
+    for (void*& u : d_u) {
+        if ((st = dalloc(&u, rsz * 6 * stride))) return st;
+        NW_TRY_HIP(hipMemsetAsync(u, 0, rsz * 6 * stride, stream));
+    }
     if (pipe == NW_PIPE_PLAIN) {
         st = init_plain(*meshes[0]);
         if (st) return st;
     } else {
-        if ((st = dalloc(&d_u[0], rsz * 6 * stride))) return st;
-        if ((st = dalloc(&d_u[1], rsz * 6 * stride))) return st;
         kchunks = 0;
         for (Segment& sg : seg) {
             sg.kbase = kchunks;
@@ -418,8 +420,6 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
             kchunks += most;
         }
         if ((st = dalloc(&d_k, ksz * 384 * kchunks))) return st;
-        NW_TRY_HIP(hipMemsetAsync(d_u[0], 0, rsz * 6 * stride, stream));
-        NW_TRY_HIP(hipMemsetAsync(d_u[1], 0, rsz * 6 * stride, stream));
         NW_TRY_HIP(hipMemsetAsync(d_k, 0, ksz * 384 * kchunks, stream));
         std::vector<int4> fnb(size_t(nelt) * 6);
         for (int r = 0; r < count; ++r) {
@@ -507,14 +507,11 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
     return NW_OK;
 }
 
-// Reference residency (dg_solver.cpp:114-236): state, k, rhs, D, w3, metrics,
-// face arrays, face scratch -- with the geometry generated on the device.
+// Reference residency (dg_solver.cpp:114-236) where the stage kernel needs it: k, D, w3,
+// metrics, face arrays -- with the geometry generated on the device.
 int Solver::init_plain(const Mesh& m) {
     int st;
-    if ((st = dalloc(reinterpret_cast<void**>(&d_state), 8 * 6 * stride))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_kk), 8 * 6 * npts))) return st;
-    if ((st = dalloc(reinterpret_cast<void**>(&d_rhs), 8 * 6 * npts))) return st;
-    NW_TRY_HIP(hipMemsetAsync(d_state, 0, 8 * 6 * stride, stream));
     NW_TRY_HIP(hipMemsetAsync(d_kk, 0, 8 * 6 * npts, stream));
     std::vector<double> Dcol(n1 * n1), w3(np);
     const GllTables& T = host_gll_tables();
@@ -534,23 +531,19 @@ int Solver::init_plain(const Mesh& m) {
     if ((st = upload_vec(&fcode, m.fcode))) return st;
     if ((st = upload_vec(&fbc, m.fbc))) return st;
     NW_TRY_HIP(launch_metrics(corners, n1, npts, d_met, stream));
-    if ((st = dalloc(reinterpret_cast<void**>(&d_vM), 4 * tfp))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_vP), 4 * tfp))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_bc), 4 * tfp))) return st;
     for (int a = 0; a < 4; ++a)
         if ((st = dalloc(reinterpret_cast<void**>(&d_face[a]), 8 * tfp))) return st;
     const double* met10[10] = {d_met[3], d_met[4], d_met[5], d_met[6],  d_met[7],
                                d_met[8], d_met[9], d_met[10], d_met[11], d_met[12]};
-    NW_TRY_HIP(launch_face_data(fcode, fbc, n1, tfp, npts, met10, d_vM, d_vP, d_bc, d_face[0], d_face[1], d_face[2],
+    NW_TRY_HIP(launch_face_data(fcode, fbc, n1, tfp, npts, met10, d_vP, d_bc, d_face[0], d_face[1], d_face[2],
                                 d_face[3], stream));
-    if ((st = dalloc(reinterpret_cast<void**>(&d_fEN), 8 * 3 * tfp))) return st;
-    if ((st = dalloc(reinterpret_cast<void**>(&d_fHN), 8 * 3 * tfp))) return st;
-    if ((st = dalloc(reinterpret_cast<void**>(&d_flux), 8 * 6 * tfp))) return st;
     if (media) {
         if ((st = upload_vec(&d_eps, m.eps))) return st;
         if ((st = upload_vec(&d_mu, m.mu_))) return st;
     }
-    kernels_per_step = 5 * (7 + (nhalo > 0 ? 2 : 0));
+    kernels_per_step = 5 * (1 + (nhalo > 0 ? 2 : 0));
     return NW_OK;
 }
 
@@ -598,7 +591,6 @@ int Solver::download(int ix, double* host, size_t n) {
 
 // Where instance I's current state lies.
 DeviceState Solver::state_of(const Instance& I) const {
-    if (pipe == NW_PIPE_PLAIN) return {d_state, true, stride, 1};
     char* u = static_cast<char*>(d_u[parity_of(I)]);
     if (prec == kFP64) return {u + 48 * I.node_base, true, 1, 6};
     return {u + 24 * I.node_base, false, 1, 6};
@@ -700,36 +692,37 @@ int Solver::enqueue_fused_stage(const StageSet& S, int s, int parity) {
     return NW_OK;
 }
 
-int Solver::enqueue_plain_stage(int s) {
-    double* st = d_state;
-    const long long S = stride;
+int Solver::enqueue_plain_stage(int s, int parity) {
+    double* uin = static_cast<double*>(d_u[parity]);
     if (nhalo > 0) {
         const int nh = static_cast<int>(nhalo);
-        NW_TRY_HIP(launch_pack<double>(st, static_cast<double*>(d_sendbuf), d_send_vol, d_off, d_sizes, nh, S, 1, stream));
+        NW_TRY_HIP(launch_pack<double>(uin, static_cast<double*>(d_sendbuf), d_send_vol, d_off, d_sizes, nh, 1, 6, stream));
         NW_TRY_HIP(hipMemcpyAsync(d_recvbuf, d_sendbuf, 8 * 6 * nhalo, hipMemcpyDeviceToDevice, stream));
+        NW_TRY_HIP(launch_unpack<double>(static_cast<const double*>(d_recvbuf), uin, d_off, d_sizes, nh, npts, 1, 6, stream));
     }
-    PlainVolumeArgs v{};
-    v.D = d_D; v.w3g = d_w3; v.jac = d_met[3];
-    v.rx = d_met[4]; v.sx = d_met[5]; v.tx = d_met[6]; v.ry = d_met[7]; v.sy = d_met[8]; v.ty = d_met[9];
-    v.rz = d_met[10]; v.sz = d_met[11]; v.tz = d_met[12];
-    v.n1 = n1; v.nelt = nelt;
-    // +curl H -> rhs_E ; -curl E -> rhs_H (dg_solver.cpp:393-413)
-    v.u1 = st + 3 * S; v.u2 = st + 4 * S; v.u3 = st + 5 * S;
-    v.w1 = d_rhs; v.w2 = d_rhs + npts; v.w3 = d_rhs + 2 * npts; v.sign = 1.0;
-    NW_TRY_HIP(launch_volume_curl(v, stream));
-    v.u1 = st; v.u2 = st + S; v.u3 = st + 2 * S;
-    v.w1 = d_rhs + 3 * npts; v.w2 = d_rhs + 4 * npts; v.w3 = d_rhs + 5 * npts; v.sign = -1.0;
-    NW_TRY_HIP(launch_volume_curl(v, stream));
-    if (nhalo > 0) {
-        NW_TRY_HIP(launch_unpack<double>(static_cast<const double*>(d_recvbuf), st, d_off, d_sizes,
-                                         static_cast<int>(nhalo), npts, S, 1, stream));
-    }
-    NW_TRY_HIP(launch_restrict(st, d_fEN, d_fHN, d_vM, tfp, S, stream));
-    NW_TRY_HIP(launch_flux(st, d_fEN, d_fHN, d_vP, d_bc, d_face[0], d_face[1], d_face[2], d_flux, c0, tfp, S, d_vM,
-                           media ? d_eps : nullptr, media ? d_mu : nullptr, d_ghost_elem, np, npts, stream));
-    NW_TRY_HIP(launch_lift(d_flux, d_face[3], d_rhs, tfp, npts, n1, stream));
-    NW_TRY_HIP(launch_inv_mass(d_rhs, d_met[3], d_w3, np, npts, media ? d_eps : nullptr, media ? d_mu : nullptr, stream));
-    NW_TRY_HIP(launch_lsrk(st, d_kk, d_rhs, kRkA[s], kRkB[s], d_dt, 0.0, npts, S, stream));
+    PlainStageArgs a{};
+    a.uin = uin;
+    a.uout = static_cast<double*>(d_u[1 - parity]);
+    a.k = d_kk;
+    a.D = d_D;
+    a.w3 = d_w3;
+    for (int m = 0; m < 10; ++m) a.met[m] = d_met[3 + m];
+    a.vP = d_vP;
+    a.bc = d_bc;
+    a.nx = d_face[0];
+    a.ny = d_face[1];
+    a.nz = d_face[2];
+    a.dA = d_face[3];
+    a.eps = media ? d_eps : nullptr;
+    a.mu = media ? d_mu : nullptr;
+    a.ghost_elem = d_ghost_elem;
+    a.dt = d_dt;
+    a.a = kRkA[s];
+    a.b = kRkB[s];
+    a.c0 = c0;
+    a.nelt = nelt;
+    a.npts = static_cast<int>(npts);
+    NW_TRY_HIP(launch_plain_stage(n1, a, stream));
     return NW_OK;
 }
 
@@ -737,19 +730,16 @@ int Solver::enqueue_step(const StageSet& S, int parity) {
     int st;
     for (int s = 0; s < kStages; ++s) {
         if (pipe == NW_PIPE_FUSED) st = enqueue_fused_stage(S, s, (parity + s) & 1);
-        else st = enqueue_plain_stage(s);
+        else st = enqueue_plain_stage(s, (parity + s) & 1);
         if (st) return st;
     }
-    // the step's result sits in d_u[parity ^ 1] (fused) or d_state (plain)
+    // the step's result sits in d_u[parity ^ 1]
     return nprobes > 0 ? enqueue_probe(parity ^ 1) : NW_OK;
 }
 
-// One probe record of the state in d_u[state_parity] (fused) or d_state (plain).
+// One probe record of the state in d_u[state_parity].
 int Solver::enqueue_probe(int state_parity) {
-    if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(launch_probe<double>(d_state, stride, 1, nprobes, d_probe_base, d_probe_w, n1, d_probe_hist,
-                                        d_probe_slot, probe_cap, stream));
-    } else if (prec == kFP64) {
+    if (prec == kFP64) {
         NW_TRY_HIP(launch_probe<double>(static_cast<const double*>(d_u[state_parity]), 1, 6, nprobes, d_probe_base,
                                         d_probe_w, n1, d_probe_hist, d_probe_slot, probe_cap, stream));
     } else {
@@ -842,7 +832,7 @@ int Solver::probe_sample() {
     if (!initialized || !uploaded) { set_error("probe_sample before create/upload"); return NW_ERR_STATE; }
     if (nprobes <= 0) { set_error("no probes set"); return NW_ERR_STATE; }
     NW_TRY_HIP(hipSetDevice(device));
-    int st = enqueue_probe(pipe == NW_PIPE_FUSED ? parity_of(inst[0]) : 0);
+    int st = enqueue_probe(parity_of(inst[0]));
     if (st) return st;
     NW_TRY_HIP(hipStreamSynchronize(stream));
     ++probe_taken;
@@ -1049,20 +1039,20 @@ int Solver::set_walk(int mode) {
     return NW_OK;
 }
 
-// nsteps steps of one set by stage launches (plain pipeline: sets[0], no segments used).
+// nsteps steps of one set by stage launches (plain pipeline: sets[0]).
 int Solver::enqueue_staged(StageSet& S, double dt, int nsteps) {
     if (nsteps <= 0) return NW_OK;
     int st = set_dt(dt);
     if (st) return st;
     for (int n = 0; n < nsteps; ++n) {
-        const int parity = (pipe == NW_PIPE_FUSED) ? S.cur : 0;
+        const int parity = S.cur;
         if (use_graph) {
             if (!S.gexec[parity] && (st = build_graph(S, parity))) return st;
             NW_TRY_HIP(hipGraphLaunch(S.gexec[parity], stream));
         } else {
             if ((st = enqueue_step(S, parity))) return st;
         }
-        if (pipe == NW_PIPE_FUSED) S.cur ^= 1;  // five stages flip the ping-pong parity
+        S.cur ^= 1;  // five stages flip the ping-pong parity
     }
     return NW_OK;
 }
@@ -1102,7 +1092,7 @@ int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
         for (int x = 0; x < 2; ++x)
             for (int p = 0; p < 2; ++p)
                 if (!sets[x].segs.empty() && !(x == 1 && resident) && !sets[x].gexec[p] &&
-                    (pipe == NW_PIPE_FUSED || p == 0) && (st = build_graph(sets[x], p))) {
+                    (st = build_graph(sets[x], p))) {
                     finish();
                     return st;
                 }
@@ -1313,12 +1303,10 @@ int Solver::diag(int ix, nw_diag* out) {
     NW_TRY_HIP(hipSetDevice(device));
     const ElemMat* mat = I.media ? d_mat + I.elem_base : nullptr;
     const ElemGeom* geom = d_geom + I.elem_base;
-    if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(launch_diag<double>(d_state, stride, 1, npts, n1, d_met[3], nullptr, mat, d_diag_part, h_page,
-                                       stream));
-    } else if (prec == kFP64) {
+    if (prec == kFP64) {
+        // d_met[3]: the plain pipeline's stored Jacobians, null in the fused one
         NW_TRY_HIP(launch_diag<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
-                                       nullptr, geom, mat, d_diag_part, h_page, stream));
+                                       d_met[3], geom, mat, d_diag_part, h_page, stream));
     } else {
         NW_TRY_HIP(launch_diag<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, I.npts, I.n1,
                                       nullptr, geom, mat, d_diag_part, h_page, stream));
@@ -1342,12 +1330,9 @@ int Solver::rel_l2(int ix, const double* ref, size_t n, double* out) {
     NW_TRY_HIP(hipSetDevice(device));
     NW_TRY_HIP(hipMemcpyAsync(d_stage, ref, 8 * 6 * I.npts, hipMemcpyHostToDevice, stream));
     const ElemGeom* geom = d_geom + I.elem_base;
-    if (pipe == NW_PIPE_PLAIN) {
-        NW_TRY_HIP(launch_l2<double>(d_state, stride, 1, d_stage, npts, n1, d_met[3], nullptr, d_diag_part, h_page,
-                                     stream));
-    } else if (prec == kFP64) {
+    if (prec == kFP64) {
         NW_TRY_HIP(launch_l2<double>(static_cast<const double*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts,
-                                     I.n1, nullptr, geom, d_diag_part, h_page, stream));
+                                     I.n1, d_met[3], geom, d_diag_part, h_page, stream));
     } else {
         NW_TRY_HIP(launch_l2<float>(static_cast<const float*>(d_u[parity_of(I)]) + 6 * I.node_base, 1, 6, d_stage, I.npts, I.n1,
                                     nullptr, geom, d_diag_part, h_page, stream));

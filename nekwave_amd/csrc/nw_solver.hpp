@@ -113,11 +113,11 @@ struct Solver {
     long long* d_snap_base = nullptr;  // per probe: its element's offset in a step's record
     int snap_slots = 0, snap_steps = 0;
     // plain pipeline (reference residency, single mesh)
-    double *d_state = nullptr, *d_kk = nullptr, *d_rhs = nullptr, *d_D = nullptr, *d_w3 = nullptr;
+    double *d_kk = nullptr, *d_D = nullptr, *d_w3 = nullptr;
     double* d_met[13] = {};  // x y z jac rx sx tx ry sy ty rz sz tz
-    int *d_vM = nullptr, *d_vP = nullptr, *d_bc = nullptr;
+    int *d_vP = nullptr, *d_bc = nullptr;
     double* d_face[4] = {};  // nx ny nz dA
-    double *d_fEN = nullptr, *d_fHN = nullptr, *d_flux = nullptr, *d_eps = nullptr, *d_mu = nullptr;
+    double *d_eps = nullptr, *d_mu = nullptr;
     // probes (device-side ProbeManager): per probe the node base of its element and
     // the 1-D Lagrange weights Lr, Ls, Lt; a history of `probe_cap` records
     int nprobes = 0, probe_cap = 0;
@@ -170,7 +170,7 @@ struct Solver {
                        bool backwards = false);
     long long working_set_bytes() const;
     int enqueue_fused_stage(const StageSet& S, int s, int parity);
-    int enqueue_plain_stage(int s);
+    int enqueue_plain_stage(int s, int parity);
     int enqueue_step(const StageSet& S, int parity);
     int build_graph(StageSet& S, int parity);
     int enqueue_probe(int state_parity);
