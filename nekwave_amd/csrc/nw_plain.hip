@@ -5,8 +5,7 @@
 // The stage kernels take the same arrays as the reference launchers
 // (dg_kernels.hpp:13-88) so every reference kernel has a counterpart that can
 // be checked in isolation.  Design differences from the reference:
-//   * volume curl: one thread per (i, j) column with the t-contraction in
-//     registers and EPW elements per workgroup (not one thread per node);
+//   * volume curl: EPW elements per workgroup, KS thread planes per element;
 //   * lift: one thread per node gathering its face contributions in face order
 //     0..5 (deterministic; the reference uses FP64 atomics, dg_kernels.cu:329);
 //   * elementwise kernels are grid-stride loops sized for 256 CUs.
@@ -32,64 +31,63 @@ inline int grid_for(long long n, int block = kBlock) {
     return static_cast<int>(g);
 }
 
+// The block's place when neighbouring blocks are to share an XCD's L2: block b runs on
+// XCD b mod 8.  The grid is a multiple of 8 (grid_for_xcd).  For the kernels that
+// gather traces, where a line of the state holds points of several blocks: flux 27.0 ->
+// 19.5 us at 593 thousand nodes, n1 = 7, 18.5 -> 14.0 at 512 thousand, n1 = 10; restrict
+// 14.6 -> 12.4 and 13.2 -> 10.3.
+inline int grid_for_xcd(long long n) { return 8 * ((grid_for(n) + 7) / 8); }
+__device__ __forceinline__ long long xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
+
 // ---------------------------------------------------------------------------
 // volume curl (dg_kernels.cu:41-155): w = sign * W*J * (grad_ref u . J^-T) x
 // ---------------------------------------------------------------------------
-template <int N1, int EPW>
-__global__ __launch_bounds__(EPW* N1* N1) void k_volume_curl(
-    const double* __restrict__ u1, const double* __restrict__ u2, const double* __restrict__ u3,
-    double* __restrict__ w1, double* __restrict__ w2, double* __restrict__ w3o,
-    const double* __restrict__ D, const double* __restrict__ w3g, const double* __restrict__ jac,
-    const double* __restrict__ rx, const double* __restrict__ sx, const double* __restrict__ tx,
-    const double* __restrict__ ry, const double* __restrict__ sy, const double* __restrict__ ty,
-    const double* __restrict__ rz, const double* __restrict__ sz, const double* __restrict__ tz,
-    double sign, int nelt) {
-    constexpr int N2 = N1 * N1, NP = N1 * N2;
+// Bound by memory: fields in and out (48 B per node) and metrics (80).  The workgroups of
+// k_plain_stage, the t-lines in LDS like the others: a thread per column with its line
+// in registers had one or two waves per element and took 24.1 us at 593 thousand nodes,
+// n1 = 7, 22.6 at 373 thousand, n1 = 8, 21.0 at 512 thousand, n1 = 10; now 16.5, 11.9
+// and 15.2 (4.3 to 4.6 TB/s).
+template <int N1, int EPW, int KS>
+__global__ __launch_bounds__(EPW* KS* N1* N1) void k_volume_curl(const PlainVolumeArgs A) {
+    constexpr int N2 = N1 * N1, NP = N1 * N2, T = KS * N2, NK = (N1 + KS - 1) / KS;
     __shared__ double sU[EPW][3][NP];
-    __shared__ double sD[N2];
-    const int tid = threadIdx.x;
-    const int es = tid / N2, l = tid - es * N2, i = l % N1, j = l / N1;
-    const int e = blockIdx.x * EPW + es;
-    const bool live = e < nelt;
-    const int ee = live ? e : nelt - 1;
-    for (int x = tid; x < N2; x += EPW * N2) sD[x] = D[x];  // column-major D[i + l*N1]
-    const long long nb = (long long)ee * NP + l;
-    double c1[N1], c2[N1], c3[N1];
+    __shared__ double sD[N2];  // column-major D[i + q * N1]
+    const int es = threadIdx.x / T, l = threadIdx.x - es * T;
+    const int ks = l / N2, ij = l - ks * N2, i = ij % N1, j = ij / N1;
+    const bool live = blockIdx.x * EPW + es < A.nelt;
+    // uniform base of the group's nodes, 32-bit offsets within it
+    const long long vg = (long long)blockIdx.x * EPW * NP;
+    const unsigned v0 = (live ? es : A.nelt - 1 - blockIdx.x * EPW) * NP;
+    for (int x = threadIdx.x; x < N2; x += EPW * T) sD[x] = A.D[x];
 #pragma unroll
-    for (int k = 0; k < N1; ++k) {
-        c1[k] = u1[nb + N2 * k]; c2[k] = u2[nb + N2 * k]; c3[k] = u3[nb + N2 * k];
-        sU[es][0][l + N2 * k] = c1[k]; sU[es][1][l + N2 * k] = c2[k]; sU[es][2][l + N2 * k] = c3[k];
+    for (int m = 0; m < NK; ++m) {
+        const int x = l + m * T;
+        if (x < NP) {
+            sU[es][0][x] = (A.u1 + vg)[v0 + x]; sU[es][1][x] = (A.u2 + vg)[v0 + x]; sU[es][2][x] = (A.u3 + vg)[v0 + x];
+        }
     }
     __syncthreads();
     if (!live) return;
 #pragma unroll
-    for (int k = 0; k < N1; ++k) {
-        double a1r = 0, a1s = 0, a1t = 0, a2r = 0, a2s = 0, a2t = 0, a3r = 0, a3s = 0, a3t = 0;
+    for (int m = 0; m < NK; ++m) {
+        const int k = ks + KS * m;
+        if (NK * KS != N1 && k >= N1) break;
+        const unsigned x = ij + N2 * k, v = v0 + x;
+        double r[3], s[3], t[3];
+        plain_gradient<N1, 3>(sU[es], sD, i, j, k, r, s, t);
+        const double* const met[9] = {A.rx, A.sx, A.tx, A.ry, A.sy, A.ty, A.rz, A.sz, A.tz};
+        double g[9];
 #pragma unroll
-        for (int q = 0; q < N1; ++q) {
-            const double di = sD[i + q * N1], dj = sD[j + q * N1], dk = sD[k + q * N1];
-            const int ir = q + N1 * j + N2 * k, is = i + N1 * q + N2 * k;
-            a1r += di * sU[es][0][ir]; a2r += di * sU[es][1][ir]; a3r += di * sU[es][2][ir];
-            a1s += dj * sU[es][0][is]; a2s += dj * sU[es][1][is]; a3s += dj * sU[es][2][is];
-            a1t += dk * c1[q]; a2t += dk * c2[q]; a3t += dk * c3[q];
-        }
-        const long long p = nb + N2 * k;
-        const double w = w3g[l + N2 * k] * jac[p];
-        const double met[9] = {rx[p], sx[p], tx[p], ry[p], sy[p], ty[p], rz[p], sz[p], tz[p]};
-        const Vec3 o = plain_curl({a1r, a2r, a3r}, {a1s, a2s, a3s}, {a1t, a2t, a3t}, w, met);
-        w1[p] = sign * o.x; w2[p] = sign * o.y; w3o[p] = sign * o.z;
+        for (int d = 0; d < 9; ++d) g[d] = (met[d] + vg)[v];
+        const Vec3 o = plain_curl(r, s, t, A.w3g[x] * (A.jac + vg)[v], g);
+        (A.w1 + vg)[v] = A.sign * o.x; (A.w2 + vg)[v] = A.sign * o.y; (A.w3 + vg)[v] = A.sign * o.z;
     }
 }
 
-constexpr int kVolEpw[kMaxN1 + 1] = {1, 1, 16, 7, 4, 2, 1, 1, 1, 1, 1};
-
 template <int N1>
 hipError_t launch_vc(const PlainVolumeArgs& a, hipStream_t s) {
-    constexpr int EPW = kVolEpw[N1];
-    const int grid = (a.nelt + EPW - 1) / EPW;
-    hipLaunchKernelGGL((k_volume_curl<N1, EPW>), dim3(grid), dim3(EPW * N1 * N1), 0, s,
-                       a.u1, a.u2, a.u3, a.w1, a.w2, a.w3, a.D, a.w3g, a.jac, a.rx, a.sx, a.tx,
-                       a.ry, a.sy, a.ty, a.rz, a.sz, a.tz, a.sign, a.nelt);
+    constexpr int EPW = PlainTile<N1>::EPW, KS = PlainTile<N1>::KS;
+    hipLaunchKernelGGL((k_volume_curl<N1, EPW, KS>), dim3((a.nelt + EPW - 1) / EPW), dim3(EPW * KS * N1 * N1), 0, s, a);
     return hipGetLastError();
 }
 
@@ -98,7 +96,7 @@ hipError_t launch_vc(const PlainVolumeArgs& a, hipStream_t s) {
 // ---------------------------------------------------------------------------
 __global__ void k_restrict(const double* __restrict__ st, double* __restrict__ fEN, double* __restrict__ fHN,
                            const int* __restrict__ vM, long long tfp, long long S) {
-    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
+    for (long long p = xcd_block() * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
         const long long v = vM[p];
         fEN[p] = st[v]; fEN[tfp + p] = st[S + v]; fEN[2 * tfp + p] = st[2 * S + v];
         fHN[p] = st[3 * S + v]; fHN[tfp + p] = st[4 * S + v]; fHN[2 * tfp + p] = st[5 * S + v];
@@ -110,7 +108,7 @@ __global__ void k_flux(const double* __restrict__ st, const double* __restrict__
                        const double* __restrict__ nya, const double* __restrict__ nza, double* __restrict__ flux,
                        double c0, long long tfp, long long S, const int* __restrict__ vM, const double* __restrict__ eps,
                        const double* __restrict__ mu, const int* __restrict__ ghost_elem, int np, long long npts) {
-    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
+    for (long long p = xcd_block() * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
         const Vec3 Em = {fEN[p], fEN[tfp + p], fEN[2 * tfp + p]}, Hm = {fHN[p], fHN[tfp + p], fHN[2 * tfp + p]};
         const int v = vP[p];
         const bool mirror = bc[p] != 0 || v < 0;
@@ -134,55 +132,70 @@ __global__ void k_flux(const double* __restrict__ st, const double* __restrict__
 }
 
 // Deterministic lift: node (i,j,k) of element e gathers dA*flux from the face
-// points that map to it, faces in order 0..5 (the serial face-point order).
-// vM == nullptr: the element-major face layout is known to hold (the solver's
-// own tables).  Otherwise a face point counts here only if volIdxMinus names the
-// node the layout puts it at; k_lift_scatter adds the others.
-__global__ void k_lift(const double* __restrict__ flux, const double* __restrict__ dA, double* __restrict__ rhs,
-                       long long tfp, long long npts, int n1, const int* __restrict__ vM) {
-    const int n2 = n1 * n1, np = n2 * n1;
-    for (long long v = blockIdx.x * (long long)blockDim.x + threadIdx.x; v < npts; v += (long long)gridDim.x * blockDim.x) {
-        const long long e = v / np;
-        const int m = static_cast<int>(v - e * np);
-        const int i = m % n1, j = (m / n1) % n1, k = m / n2;
-        int pts[6], nf = 0;
-        const long long fb = e * 6 * n2;
-        if (j == 0) pts[nf++] = 0 * n2 + i + n1 * k;
-        if (i == n1 - 1) pts[nf++] = 1 * n2 + j + n1 * k;
-        if (j == n1 - 1) pts[nf++] = 2 * n2 + i + n1 * k;
-        if (i == 0) pts[nf++] = 3 * n2 + j + n1 * k;
-        if (k == 0) pts[nf++] = 4 * n2 + i + n1 * j;
-        if (k == n1 - 1) pts[nf++] = 5 * n2 + i + n1 * j;
-        if (nf == 0) continue;
-        double r0 = rhs[v], r1 = rhs[npts + v], r2 = rhs[2 * npts + v];
-        double r3 = rhs[3 * npts + v], r4 = rhs[4 * npts + v], r5 = rhs[5 * npts + v];
-        for (int t = 0; t < nf; ++t) {
+// points that map to it, faces in order 0..5 (the serial face-point order).  A
+// face point counts here only if volIdxMinus names the node the element-major
+// layout puts it at; k_lift_scatter adds the others.  A node lies on at most one
+// face per axis: the reads of its (up to) three points are issued together, the
+// additions follow in face order.  (With k_lift_scatter 22.8 us at 593 thousand
+// nodes, n1 = 7, 14.6 at 373 thousand, n1 = 8, 32.2 at 512 thousand, n1 = 2; as a loop
+// over the node's faces, each read waiting for the last and n1 a variable, 24.9, 16.2
+// and 45.0.)
+template <int N1>
+__global__ __launch_bounds__(kBlock) void k_lift(const double* __restrict__ flux, const double* __restrict__ dA,
+                                                 double* __restrict__ rhs, long long tfp, long long npts,
+                                                 const int* __restrict__ vM) {
+    constexpr int N2 = N1 * N1, NP = N2 * N1;
+    for (long long v = blockIdx.x * (long long)kBlock + threadIdx.x; v < npts; v += (long long)gridDim.x * kBlock) {
+        const unsigned e = unsigned(v) / NP;  // volIdxMinus is 32-bit, so v is
+        const int m = static_cast<int>(unsigned(v) - e * NP);
+        const int i = m % N1, j = (m / N1) % N1, k = m / N2;
+        const int pj = j == 0 ? i + N1 * k : (j == N1 - 1 ? 2 * N2 + i + N1 * k : -1);
+        const int pi = i == N1 - 1 ? N2 + j + N1 * k : (i == 0 ? 3 * N2 + j + N1 * k : -1);
+        const int pk = k == 0 ? 4 * N2 + i + N1 * j : (k == N1 - 1 ? 5 * N2 + i + N1 * j : -1);
+        const bool j_first = pj >= 0 && (pi < 0 || pj < pi);
+        const int pts[3] = {j_first ? pj : pi, j_first ? pi : pj, pk};
+        if (pj < 0 && pi < 0 && pk < 0) continue;
+        const long long fb = (long long)e * 6 * N2;
+        double a[3], f[3][6], r[6];
+        bool on[3];
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
             const long long p = fb + pts[t];
-            if (vM && vM[p] != v) continue;
-            const double a = dA[p];
-            r0 += a * flux[3 * tfp + p]; r1 += a * flux[4 * tfp + p]; r2 += a * flux[5 * tfp + p];
-            r3 += a * flux[p]; r4 += a * flux[tfp + p]; r5 += a * flux[2 * tfp + p];
+            on[t] = pts[t] >= 0 && vM[p] == v;
+            if (pts[t] >= 0) {
+                a[t] = dA[p];
+#pragma unroll
+                for (int c = 0; c < 6; ++c) f[t][c] = flux[(c < 3 ? c + 3 : c - 3) * tfp + p];
+            }
         }
-        rhs[v] = r0; rhs[npts + v] = r1; rhs[2 * npts + v] = r2;
-        rhs[3 * npts + v] = r3; rhs[4 * npts + v] = r4; rhs[5 * npts + v] = r5;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) r[c] = rhs[c * npts + v];
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            if (on[t]) {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) r[c] += a[t] * f[t][c];
+            }
+#pragma unroll
+        for (int c = 0; c < 6; ++c) rhs[c * npts + v] = r[c];
     }
 }
 
-// The face points k_lift did not take (n1 > 0: those whose volIdxMinus is not
-// the node the element-major layout puts them at; n1 == 0: all of them), added
+// The face points k_lift did not take (N1 > 0: those whose volIdxMinus is not
+// the node the element-major layout puts them at; N1 == 0: all of them), added
 // as the reference adds every point: rhs[vM] += dA * flux with FP64 atomics
 // (dg_kernels.cu:316-338).  Points with vM outside [0, npts) are skipped.
-__global__ void k_lift_scatter(const double* __restrict__ flux, const double* __restrict__ dA, double* __restrict__ rhs,
-                               long long tfp, long long npts, int n1, const int* __restrict__ vM) {
-    const int n2 = n1 * n1, nf2 = 6 * n2;
-    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < tfp; p += (long long)gridDim.x * blockDim.x) {
+template <int N1>
+__global__ __launch_bounds__(kBlock) void k_lift_scatter(const double* __restrict__ flux, const double* __restrict__ dA,
+                                                         double* __restrict__ rhs, long long tfp, long long npts,
+                                                         const int* __restrict__ vM) {
+    for (long long p = blockIdx.x * (long long)kBlock + threadIdx.x; p < tfp; p += (long long)gridDim.x * kBlock) {
         const long long v = vM[p];
-        if (n1 > 0) {
-            const long long e = p / nf2;
-            const int r = static_cast<int>(p - e * nf2), f = r / n2, pq = r - f * n2;
-            int i, j, k;
-            face_ijk(f, n1, pq % n1, pq / n1, i, j, k);
-            if (v == e * n2 * n1 + i + n1 * (j + n1 * k)) continue;
+        if constexpr (N1 > 0) {
+            constexpr int N2 = N1 * N1;
+            const long long e = p / (6 * N2);
+            const int r = static_cast<int>(p - e * 6 * N2), f = r / N2, pq = r - f * N2;
+            if (v == e * N2 * N1 + face_local_node<N1>(f, pq % N1, pq / N1)) continue;
         }
         if (v < 0 || v >= npts) continue;
         const double a = dA[p];
@@ -195,14 +208,22 @@ __global__ void k_lift_scatter(const double* __restrict__ flux, const double* __
     }
 }
 
+template <int N1>
+void launch_lifts(const double* flux, const double* dA, double* rhs, long long tfp, long long npts, const int* vM,
+                  hipStream_t s) {
+    if constexpr (N1 > 0)
+        hipLaunchKernelGGL(k_lift<N1>, dim3(grid_for(npts)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, vM);
+    hipLaunchKernelGGL(k_lift_scatter<N1>, dim3(grid_for(tfp)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, vM);
+}
+
 __global__ void k_inv_mass(double* __restrict__ rhs, const double* __restrict__ jac, const double* __restrict__ w3,
                            int nxyz, long long npts, const double* __restrict__ eps, const double* __restrict__ mu) {
     for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < npts; idx += (long long)gridDim.x * blockDim.x) {
-        const long long e = idx / nxyz;
+        const long long e = npts <= 0x7fffffff ? unsigned(idx) / unsigned(nxyz) : idx / nxyz;
         const int i = static_cast<int>(idx - e * nxyz);
-        const double ep = eps ? eps[e] : 1.0, m = mu ? mu[e] : 1.0;
+        const double ep = eps ? eps[e] : 1.0;
         const double iE = 1.0 / (ep * jac[idx] * w3[i]);
-        const double iH = 1.0 / (m * jac[idx] * w3[i]);
+        const double iH = eps || mu ? 1.0 / ((mu ? mu[e] : 1.0) * jac[idx] * w3[i]) : iE;
         rhs[idx] *= iE; rhs[npts + idx] *= iE; rhs[2 * npts + idx] *= iE;
         rhs[3 * npts + idx] *= iH; rhs[4 * npts + idx] *= iH; rhs[5 * npts + idx] *= iH;
     }
@@ -210,12 +231,11 @@ __global__ void k_inv_mass(double* __restrict__ rhs, const double* __restrict__ 
 
 __global__ void k_lsrk(double* __restrict__ st, double* __restrict__ k, const double* __restrict__ rhs, double a,
                        double b, double dt, long long npts, long long S) {
-    const long long n = 6 * npts;
-    for (long long x = blockIdx.x * (long long)blockDim.x + threadIdx.x; x < n; x += (long long)gridDim.x * blockDim.x) {
-        const long long c = x / npts, p = x - c * npts;
-        const double ki = a * k[x] + dt * rhs[x];
-        k[x] = ki;
-        st[c * S + p] += b * ki;
+    const long long base = blockIdx.y * npts, sb = blockIdx.y * S;  // one component per grid row
+    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < npts; p += (long long)gridDim.x * blockDim.x) {
+        const double ki = a * k[base + p] + dt * rhs[base + p];
+        k[base + p] = ki;
+        st[sb + p] += b * ki;
     }
 }
 
@@ -645,7 +665,7 @@ hipError_t launch_volume_curl(const PlainVolumeArgs& a, hipStream_t s) {
 hipError_t launch_restrict(const double* st, double* fEN, double* fHN, const int* vM, long long tfp, long long S,
                            hipStream_t s) {
     if (tfp <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_restrict, dim3(grid_for(tfp)), dim3(kBlock), 0, s, st, fEN, fHN, vM, tfp, S);
+    hipLaunchKernelGGL(k_restrict, dim3(grid_for_xcd(tfp)), dim3(kBlock), 0, s, st, fEN, fHN, vM, tfp, S);
     return hipGetLastError();
 }
 
@@ -654,7 +674,7 @@ hipError_t launch_flux(const double* st, const double* fEN, const double* fHN, c
                        long long S, const int* vM, const double* eps, const double* mu, const int* ghost_elem, int np,
                        long long npts, hipStream_t s) {
     if (tfp <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_flux, dim3(grid_for(tfp)), dim3(kBlock), 0, s, st, fEN, fHN, vP, bc, nx, ny, nz, flux, c0,
+    hipLaunchKernelGGL(k_flux, dim3(grid_for_xcd(tfp)), dim3(kBlock), 0, s, st, fEN, fHN, vP, bc, nx, ny, nz, flux, c0,
                        tfp, S, vM, eps, mu, ghost_elem, np, npts);
     return hipGetLastError();
 }
@@ -670,12 +690,18 @@ hipError_t launch_add_flux(const double* flux, const int* vM, const double* dA, 
         if (c >= kMinN1 && c <= kMaxN1 && npts % (c * c * c) == 0 && tfp == 6 * c * c * (npts / (c * c * c)))
             n1 = static_cast<int>(c);
     }
-    if (n1 > 0) {
-        hipLaunchKernelGGL(k_lift, dim3(grid_for(npts)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, n1, vM);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+    switch (n1) {
+        case 2: launch_lifts<2>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 3: launch_lifts<3>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 4: launch_lifts<4>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 5: launch_lifts<5>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 6: launch_lifts<6>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 7: launch_lifts<7>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 8: launch_lifts<8>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 9: launch_lifts<9>(flux, dA, rhs, tfp, npts, vM, s); break;
+        case 10: launch_lifts<10>(flux, dA, rhs, tfp, npts, vM, s); break;
+        default: launch_lifts<0>(flux, dA, rhs, tfp, npts, vM, s); break;
     }
-    hipLaunchKernelGGL(k_lift_scatter, dim3(grid_for(tfp)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, n1, vM);
     return hipGetLastError();
 }
 
@@ -689,7 +715,7 @@ hipError_t launch_inv_mass(double* rhs, const double* jac, const double* w3, int
 hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, double dt,
                        long long npts, long long S, hipStream_t s) {
     if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_lsrk, dim3(grid_for(6 * npts)), dim3(kBlock), 0, s, st, k, rhs, a, b, dt, npts, S);
+    hipLaunchKernelGGL(k_lsrk, dim3(grid_for(npts), 6), dim3(kBlock), 0, s, st, k, rhs, a, b, dt, npts, S);
     return hipGetLastError();
 }
 

@@ -8,9 +8,55 @@
 namespace nw {
 namespace {
 
+// Elements per workgroup and thread planes per element.  The workgroups of a CU cover
+// each other's barriers and loads: at n1 = 10 five planes of two nodes per thread (500
+// threads, 110 registers, two workgroups per CU) take 31.1 us, ten planes (1000 threads,
+// one workgroup) 34.8; n1 = 9 27.1 against 28.5; n1 = 8 four planes 26.2 against 27.9; from
+// n1 = 7 down one node per thread.  Small elements: about two waves per workgroup (n1 = 5
+// one element 26.3, two 26.9, four 29.0).
+template <int N1> struct PlainTile;
+template <> struct PlainTile<2> { static constexpr int EPW = 16, KS = 2; };
+template <> struct PlainTile<3> { static constexpr int EPW = 4, KS = 3; };
+template <> struct PlainTile<4> { static constexpr int EPW = 2, KS = 4; };
+template <> struct PlainTile<5> { static constexpr int EPW = 1, KS = 5; };
+template <> struct PlainTile<6> { static constexpr int EPW = 1, KS = 6; };
+template <> struct PlainTile<7> { static constexpr int EPW = 1, KS = 7; };
+template <> struct PlainTile<8> { static constexpr int EPW = 1, KS = 4; };
+template <> struct PlainTile<9> { static constexpr int EPW = 1, KS = 5; };
+template <> struct PlainTile<10> { static constexpr int EPW = 1, KS = 5; };
+
+// Local node of face point (p, q) of face f, without branches.
+template <int N1>
+__device__ __forceinline__ int face_local_node(int f, int p, int q) {
+    constexpr int N2 = N1 * N1;
+    const int base = f == 1 ? N1 - 1 : f == 2 ? N1 * (N1 - 1) : f == 5 ? N2 * (N1 - 1) : 0;
+    return base + p * ((f == 1 || f == 3) ? N1 : 1) + q * (f >= 4 ? N1 : N2);
+}
+
 struct Vec3 {
     double x, y, z;
 };
+
+// Derivatives along the reference axes of NC fields at node (i, j, k) of the element in
+// u, from the column-major D.  (q rolled: unrolled, the reads ahead of their use take
+// the registers of a second workgroup per CU.)
+template <int N1, int NC>
+__device__ __forceinline__ void plain_gradient(const double (&u)[NC][N1 * N1 * N1], const double* sD, int i, int j, int k,
+                                               double (&r)[NC], double (&s)[NC], double (&t)[NC]) {
+    constexpr int N2 = N1 * N1;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) r[c] = s[c] = t[c] = 0.0;
+#pragma unroll 1
+    for (int q = 0; q < N1; ++q) {
+        const double di = sD[i + q * N1], dj = sD[j + q * N1], dk = sD[k + q * N1];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            r[c] += di * u[c][q + N1 * j + N2 * k];
+            s[c] += dj * u[c][i + N1 * q + N2 * k];
+            t[c] += dk * u[c][i + N1 * j + N2 * q];
+        }
+    }
+}
 
 // W J (grad_ref u . J^-T) x of one node (dg_kernels.cu:106-154): r, s, t the derivatives
 // of the three components along the reference axes, w = W J.

@@ -27,23 +27,6 @@
 namespace nw {
 namespace {
 
-// Elements per workgroup and thread planes per element.  The workgroups of a CU cover
-// each other's barriers and loads: at n1 = 10 five planes of two nodes per thread (500
-// threads, 110 registers, two workgroups per CU) take 31.1 us, ten planes (1000 threads,
-// one workgroup) 34.8; n1 = 9 27.1 against 28.5; n1 = 8 four planes 26.2 against 27.9; from
-// n1 = 7 down one node per thread.  Small elements: about two waves per workgroup (n1 = 5
-// one element 26.3, two 26.9, four 29.0).
-template <int N1> struct PlainTile;
-template <> struct PlainTile<2> { static constexpr int EPW = 16, KS = 2; };
-template <> struct PlainTile<3> { static constexpr int EPW = 4, KS = 3; };
-template <> struct PlainTile<4> { static constexpr int EPW = 2, KS = 4; };
-template <> struct PlainTile<5> { static constexpr int EPW = 1, KS = 5; };
-template <> struct PlainTile<6> { static constexpr int EPW = 1, KS = 6; };
-template <> struct PlainTile<7> { static constexpr int EPW = 1, KS = 7; };
-template <> struct PlainTile<8> { static constexpr int EPW = 1, KS = 4; };
-template <> struct PlainTile<9> { static constexpr int EPW = 1, KS = 5; };
-template <> struct PlainTile<10> { static constexpr int EPW = 1, KS = 5; };
-
 struct Node6 {
     double c[6];
 };
@@ -55,14 +38,6 @@ __device__ __forceinline__ Node6 load_node(const double* __restrict__ u, I v) {
 }
 
 __device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
-
-// Local node of face point (p, q) of face f, without branches.
-template <int N1>
-__device__ __forceinline__ int face_local_node(int f, int p, int q) {
-    constexpr int N2 = N1 * N1;
-    const int base = f == 1 ? N1 - 1 : f == 2 ? N1 * (N1 - 1) : f == 5 ? N2 * (N1 - 1) : 0;
-    return base + p * ((f == 1 || f == 3) ? N1 : 1) + q * (f >= 4 ? N1 : N2);
-}
 
 struct FacePoint {
     int v;  // plus node
@@ -147,25 +122,16 @@ __global__ __launch_bounds__(EPW* KS* N1* N1) void k_plain_stage(const PlainStag
     }
 
     // volume: +curl H into the rows of E, -curl E into the rows of H
-    // (q rolled: unrolled, the reads ahead of their use take the registers of the second
-    // workgroup; metrics and k read ahead of this loop did too, 34.2 -> 42.3 us at n1 = 10)
+    // (metrics and k read ahead of this loop take the registers of the second workgroup:
+    // 34.2 -> 42.3 us at n1 = 10)
     double rhs[NK][6];
 #pragma unroll
     for (int m = 0; m < NK; ++m) {
         const int k = NK * KS == N1 ? ks + KS * m : min(ks + KS * m, N1 - 1);
         const int x = ij + N2 * k;
         const unsigned v = v0 + x;
-        double ar[6] = {}, as[6] = {}, at[6] = {};
-#pragma unroll 1
-        for (int q = 0; q < N1; ++q) {
-            const double di = sD[i + q * N1], dj = sD[j + q * N1], dk = sD[k + q * N1];
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                ar[c] += di * sU[es][c][q + N1 * j + N2 * k];
-                as[c] += dj * sU[es][c][i + N1 * q + N2 * k];
-                at[c] += dk * sU[es][c][ij + N2 * q];
-            }
-        }
+        double ar[6], as[6], at[6];
+        plain_gradient<N1, 6>(sU[es], sD, i, j, k, ar, as, at);
         double met[9];
 #pragma unroll
         for (int d = 0; d < 9; ++d) met[d] = (A.met[1 + d] + vg)[v];
