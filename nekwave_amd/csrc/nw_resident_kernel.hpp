@@ -11,11 +11,43 @@
 namespace nw {
 namespace {
 
-// LDS bytes of one workgroup, as k_resident declares them.
+// LDS bytes of one workgroup, as k_resident declares them, without LSRK registers.
 constexpr int resident_lds(int n1, int em, int rsz, bool affine) {
     const int n2 = n1 * n1;
     const int plane = n1 == 8 && rsz == 4 ? 72 : n2, sent = n1 == 8 && rsz == 4 ? 1 : 0;
     return rsz * ((em + sent) * 6 * plane * n1 + (6 * n2 + 1) * 6 + n2 + n1 + em * (affine ? 12 : 26)) + 32;
+}
+// VGPRs a thread may have, and the workgroups per CU that they and LDS allow.
+template <int NT, int RBYTES>
+constexpr int resident_budget() {
+    constexpr int waves = (NT + 63) / 64, eu = WavesPerEU<NT, RBYTES>::value, own = (waves + 3) / 4;
+    return 512 / (eu > own ? eu : own) / 8 * 8;
+}
+template <int NT, int RBYTES>
+constexpr int resident_fit(int lds) {
+    constexpr int waves = (NT + 63) / 64, eu = WavesPerEU<NT, RBYTES>::value;
+    constexpr int regs = 4 * eu / waves > 1 ? 4 * eu / waves : 1;
+    return regs < 160 * 1024 / lds ? regs : 160 * 1024 / lds;
+}
+// Elements whose LSRK registers lie in LDS instead of VGPRs: enough that nothing spills (a
+// reload inside the stage waits for every packet in flight), as far as they fit beside
+// the fields without costing a workgroup per CU.  The need is what the compiler reports
+// for kernels that do not spill: a base by face points per thread, field type and
+// geometry, and per element its LSRK registers and packet offsets.  Measured per stage,
+// all in VGPRs -> this: FP32 jittered n1 = 5, 2744 elements 14.9 -> 10.9 us; FP64 jittered
+// n1 = 5, 1000 13.6 -> 9.6; FP32 with FP64 registers jittered n1 = 7, 1287 16.8 -> 15.1,
+// n1 = 5, 1728 10.2 -> 7.9.  Where nothing spills LDS costs 1-3 % (n1 = 9, 1000 elements
+// 16.2 -> 16.5), so the registers stay there.
+template <int N1, int EM, int RBYTES, int KBYTES, bool AFF>
+constexpr int resident_lds_k() {
+    constexpr int NT = N1 * N1 * N1, fpt = (6 * N1 * N1 + NT - 1) / NT, kregs = 6 * KBYTES / 4;
+    constexpr int base = fpt == 1 ? (RBYTES == 4 ? (AFF ? 98 : 112) : (AFF ? 147 : 190))
+                                  : (RBYTES == 4 ? (AFF ? 106 : 151) : (AFF ? 182 : 272));
+    constexpr int lds = resident_lds(N1, EM, RBYTES, AFF), per = 6 * NT * KBYTES, budget = resident_budget<NT, RBYTES>();
+    int n = 0;
+    while (EM > 1 && n < EM && base + EM * fpt + (EM - n) * kregs > budget && lds + (n + 1) * per <= 160 * 1024 &&
+           resident_fit<NT, RBYTES>(lds + (n + 1) * per) >= resident_fit<NT, RBYTES>(lds)) ++n;
+    return n;
 }
 
 // A uniform base and a 32-bit offset per lane: no 64-bit address arithmetic.
@@ -71,6 +103,12 @@ void k_resident(ResidentArgs A) {
     __shared__ R sZ[N1];         // GLL nodes
     __shared__ R sG[EM][GW];
     __shared__ R sM[EM][2];      // 1/eps, 1/mu
+    constexpr int KL = resident_lds_k<N1, EM, sizeof(R), sizeof(KR), AFF>();
+    // LSRK registers of elements 0 .. KL - 1, [element][component][node].  Dynamic LDS: as
+    // static LDS it would count in the compiler's occupancy, which then spends the
+    // registers of a second workgroup
+    extern __shared__ double sKdyn[];
+    KR* const sK = reinterpret_cast<KR*>(sKdyn);
     __shared__ int sStop;
 
     const int tid = threadIdx.x, m = tid;
@@ -147,17 +185,16 @@ void k_resident(ResidentArgs A) {
         }
     };
 
-    // Per element: LSRK registers, and the byte offset of the plus side's packets of
-    // the thread's face points (-1: mirror; the exchange buffer is below 2 GiB, the
-    // launcher's limit).  The element in hand has them in kc and slot; the others
+    // Per element: LSRK registers (in LDS for the first KL), and the byte offset of the
+    // plus side's packets of the thread's face points (-1: mirror; the exchange buffer is
+    // below 2 GiB, the launcher's limit).  The element in hand has them in kc and slot; the others
     // stay in registers, moved by uniform branches (pinned: as selects, every
     // element would cost moves of all of them).
-    KR kk[EM][6], kc[6];
+    KR kk[EM > KL ? EM - KL : 1][6], kc[6];
     int slots[EM][FPT], slot[FPT];
 #pragma unroll
     for (int x = 0; x < EM; ++x) {
-#pragma unroll
-        for (int c = 0; c < 6; ++c) kk[x][c] = KR(0);
+        for (int c = 0; c < 6 && x >= KL; ++c) kk[x - KL][c] = KR(0);
 #pragma unroll
         for (int t = 0; t < FPT; ++t) {
             slots[x][t] = -1;
@@ -177,23 +214,29 @@ void k_resident(ResidentArgs A) {
             }
     };
     // taken at the update (six registers fewer live through the volume work: n1 = 8,
-    // 1728 jittered elements 18.5 against 20.4 us per stage); FP64 registers under FP32
-    // fields spill either way and are taken first (n1 = 7, 1287 elements: 17.3 against 18.4)
-    constexpr bool K_EARLY = sizeof(KR) != sizeof(R);
+    // 1728 jittered elements 18.5 against 20.4 us per stage)
     auto take_k = [&](int x) {
+        if (KL > 0 && x < KL) {
 #pragma unroll
-        for (int y = 0; y < EM; ++y)
+            for (int c = 0; c < 6; ++c) kc[c] = sK[(x * 6 + c) * NP + m];
+        }
+#pragma unroll
+        for (int y = KL; y < EM; ++y)
             if (EM == 1 || x == y) {
 #pragma unroll
-                for (int c = 0; c < 6; ++c) { kc[c] = kk[y][c]; if (EM > 1) pin(kc[c]); }
+                for (int c = 0; c < 6; ++c) { kc[c] = kk[y - KL][c]; if (EM > 1) pin(kc[c]); }
             }
     };
     auto keep_k = [&](int x) {
+        if (KL > 0 && x < KL) {
 #pragma unroll
-        for (int y = 0; y < EM; ++y)
+            for (int c = 0; c < 6; ++c) sK[(x * 6 + c) * NP + m] = kc[c];
+        }
+#pragma unroll
+        for (int y = KL; y < EM; ++y)
             if (EM == 1 || x == y) {
 #pragma unroll
-                for (int c = 0; c < 6; ++c) { kk[y][c] = kc[c]; if (EM > 1) pin(kk[y][c]); }
+                for (int c = 0; c < 6; ++c) { kk[y - KL][c] = kc[c]; if (EM > 1) pin(kk[y - KL][c]); }
             }
     };
 
@@ -317,7 +360,6 @@ void k_resident(ResidentArgs A) {
 #pragma unroll 1
             for (int x = 0; x < (KEEP ? 1 : cnt); ++x) {
                 take_slots(x);
-                if constexpr (K_EARLY) take_k(x);
                 // With several elements per workgroup a neighbour's traces were mostly
                 // published an element or more ago: they are read before the volume
                 // work, which hides their latency.  Else in the middle of it.
@@ -465,7 +507,7 @@ void k_resident(ResidentArgs A) {
                         LE[c] = (sF[sj][c] + sF[si][c]) + sF[sk][c];
                         LH[c] = (sF[sj][c + 3] + sF[si][c + 3]) + sF[sk][c + 3];
                     }
-                    if constexpr (!K_EARLY) take_k(x);
+                    take_k(x);
                     const R iJ = geo[9];
                     const R sE_ = sM[x][0] * iJ, sH_ = sM[x][1] * iJ;
 #pragma unroll
@@ -500,9 +542,10 @@ void k_resident(ResidentArgs A) {
 
 template <int N1, int EM, typename R, typename KR, bool AFF>
 struct ResidentFamily {
+    static constexpr int lds_k = resident_lds_k<N1, EM, sizeof(R), sizeof(KR), AFF>() * 6 * N1 * N1 * N1 * int(sizeof(KR));
     static hipError_t launch(const ResidentArgs& a, hipStream_t s) {
         const int grid = (a.nelt + a.per - 1) / a.per;
-        hipLaunchKernelGGL((k_resident<N1, EM, R, KR, AFF>), dim3(grid), dim3(N1 * N1 * N1), 0, s, a);
+        hipLaunchKernelGGL((k_resident<N1, EM, R, KR, AFF>), dim3(grid), dim3(N1 * N1 * N1), lds_k, s, a);
         return hipGetLastError();
     }
     // Workgroups per CU that the hardware places wherever its waves start: the
@@ -515,7 +558,7 @@ struct ResidentFamily {
         if (n >= 0) return n;
         hipFuncAttributes fa;
         const void* fn = reinterpret_cast<const void*>(&k_resident<N1, EM, R, KR, AFF>);
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_resident<N1, EM, R, KR, AFF>, N1 * N1 * N1, 0) != hipSuccess ||
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_resident<N1, EM, R, KR, AFF>, N1 * N1 * N1, lds_k) != hipSuccess ||
             hipFuncGetAttributes(&fa, fn) != hipSuccess)
             return 0;
         constexpr int W = (N1 * N1 * N1 + 63) / 64;
