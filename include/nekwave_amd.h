@@ -44,7 +44,8 @@ enum {
  * FP32's (relative L2 against FP64 <= 1e-4 after 1000 steps of the 16^3
  * workload, against 1e-5 for FP32). */
 enum { NW_PREC_FP64 = 0, NW_PREC_FP32 = 1, NW_PREC_FP32_K64 = 2, NW_PREC_BF16X3 = 3 };
-/* NW_PIPE_PLAIN: the reference's 7-kernel stage (dg_solver.cpp:393-505), FP64 only.
+/* NW_PIPE_PLAIN: the reference's stage (dg_solver.cpp:393-505) from its stored per-node
+ * and per-face-point geometry, one launch per stage, FP64 only.
  * NW_PIPE_FUSED: one fused kernel per stage. */
 enum { NW_PIPE_PLAIN = 0, NW_PIPE_FUSED = 1 };
 /* face kinds: the bcType strings of FaceInfo (mesh.hpp:15-21, mesh.cpp:730-830) */

@@ -63,7 +63,7 @@ __device__ __forceinline__ unsigned long long packet_load(const char* base, unsi
 // One launch = nsteps LSRK45 steps of the elements of `nelt`, all on chip at once: a
 // workgroup owns up to EM elements, one thread per node (as k_fused_stage with one
 // element per workgroup, whose expressions it repeats: the same bits), fields in
-// LDS, LSRK registers in VGPRs.  HBM is touched at the launch's ends only; per stage
+// LDS, LSRK registers in VGPRs (or LDS: resident_lds_k).  HBM is touched at the launch's ends only; per stage
 // an element's six traces go out and its neighbours' come in.
 //
 // Why: a stage of a small mesh is bound by its launch (3-4 us for dispatch and the
@@ -72,16 +72,17 @@ __device__ __forceinline__ unsigned long long packet_load(const char* base, unsi
 // flux -> two barriers.  Measured per stage, stage launches against this kernel:
 //   n1 = 5,   64 elements, FP64              6.7 ->  2.6 us
 //   n1 = 8,  216 / 512 elements, FP32        7.6 ->  2.7 / 10.5 -> 4.2 us
-//   n1 = 6, 1000 elements, FP64             14.5 ->  8.9 us
-//   n1 = 8, 1728 elements, FP32             22.7 -> 14.0 us (uniform), 23.7 -> 18.5 us (jittered)
+//   n1 = 6, 1000 elements, FP64             14.5 ->  9.6 us
+//   n1 = 8, 1728 elements, FP32             21.6 -> 15.4 us (uniform), 23.7 -> 18.6 us (jittered)
 //   n1 = 9, 1728 elements, FP32, jittered   37.9 -> 29.0 us
-//   n1 = 4, 5832 elements, FP32             12.0 ->  8.3 us
+//   n1 = 4, 5832 elements, FP32             12.0 ->  8.2 us
 // Up to one element per workgroup the stage is bound by that chain (packets alone:
 // 1.3 us for 64 workgroups, 2.5 for 256, 4.3 for 512 at 384 points each); beyond, by
 // the vector ALUs (54-60 % busy) and LDS (55-60 %; n1 = 8 in FP32 77 % before QB).
 // Traces as plain values behind a per-wave flag (half the bytes) were slower
 // everywhere (n1 = 8, 512 elements 6.0 us, 1728 elements 17.9): two trips of the
-// fabric instead of one.
+// fabric instead of one.  So were packets stored by a node's own thread at once after its
+// update (partly filled waves: 512 elements 5.1).
 template <int N1, int EM, typename R, typename KR, bool AFF>
 __global__ __launch_bounds__(N1* N1* N1) __attribute__((amdgpu_waves_per_eu(WavesPerEU<N1 * N1 * N1, sizeof(R)>::value)))
 void k_resident(ResidentArgs A) {
