@@ -35,7 +35,9 @@ inline int grid_for(long long n, int block = kBlock) {
 // XCD b mod 8.  The grid is a multiple of 8 (grid_for_xcd).  For the kernels that
 // gather traces, where a line of the state holds points of several blocks: flux 27.0 ->
 // 19.5 us at 593 thousand nodes, n1 = 7, 18.5 -> 14.0 at 512 thousand, n1 = 10; restrict
-// 14.6 -> 12.4 and 13.2 -> 10.3.
+// 14.6 -> 12.4 and 13.2 -> 10.3.  For the kernels over nodes too: each then finds lines
+// of the one before it in its L2 (a stage 104.4 -> 101.0 at n1 = 7, 68.2 -> 64.8 at 373
+// thousand, n1 = 8, 80.2 -> 75.2 at 373 thousand, n1 = 4).
 inline int grid_for_xcd(long long n) { return 8 * ((grid_for(n) + 7) / 8); }
 __device__ __forceinline__ long long xcd_block() { return (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3); }
 
@@ -54,10 +56,12 @@ __global__ __launch_bounds__(EPW* KS* N1* N1) void k_volume_curl(const PlainVolu
     __shared__ double sD[N2];  // column-major D[i + q * N1]
     const int es = threadIdx.x / T, l = threadIdx.x - es * T;
     const int ks = l / N2, ij = l - ks * N2, i = ij % N1, j = ij / N1;
-    const bool live = blockIdx.x * EPW + es < A.nelt;
+    const int group = static_cast<int>(xcd_block());
+    if (group * EPW >= A.nelt) return;
+    const bool live = group * EPW + es < A.nelt;
     // uniform base of the group's nodes, 32-bit offsets within it
-    const long long vg = (long long)blockIdx.x * EPW * NP;
-    const unsigned v0 = (live ? es : A.nelt - 1 - blockIdx.x * EPW) * NP;
+    const long long vg = (long long)group * EPW * NP;
+    const unsigned v0 = (live ? es : A.nelt - 1 - group * EPW) * NP;
     for (int x = threadIdx.x; x < N2; x += EPW * T) sD[x] = A.D[x];
 #pragma unroll
     for (int m = 0; m < NK; ++m) {
@@ -87,7 +91,8 @@ __global__ __launch_bounds__(EPW* KS* N1* N1) void k_volume_curl(const PlainVolu
 template <int N1>
 hipError_t launch_vc(const PlainVolumeArgs& a, hipStream_t s) {
     constexpr int EPW = PlainTile<N1>::EPW, KS = PlainTile<N1>::KS;
-    hipLaunchKernelGGL((k_volume_curl<N1, EPW, KS>), dim3((a.nelt + EPW - 1) / EPW), dim3(EPW * KS * N1 * N1), 0, s, a);
+    const int groups = (a.nelt + EPW - 1) / EPW;
+    hipLaunchKernelGGL((k_volume_curl<N1, EPW, KS>), dim3(8 * ((groups + 7) / 8)), dim3(EPW * KS * N1 * N1), 0, s, a);
     return hipGetLastError();
 }
 
@@ -136,8 +141,8 @@ __global__ void k_flux(const double* __restrict__ st, const double* __restrict__
 // face point counts here only if volIdxMinus names the node the element-major
 // layout puts it at; k_lift_scatter adds the others.  A node lies on at most one
 // face per axis: the reads of its (up to) three points are issued together, the
-// additions follow in face order.  (With k_lift_scatter 22.8 us at 593 thousand
-// nodes, n1 = 7, 14.6 at 373 thousand, n1 = 8, 32.2 at 512 thousand, n1 = 2; as a loop
+// additions follow in face order.  (With k_lift_scatter 21.2 us at 593 thousand
+// nodes, n1 = 7, 14.9 at 373 thousand, n1 = 8, 32.9 at 512 thousand, n1 = 2; as a loop
 // over the node's faces, each read waiting for the last and n1 a variable, 24.9, 16.2
 // and 45.0.)
 template <int N1>
@@ -145,7 +150,7 @@ __global__ __launch_bounds__(kBlock) void k_lift(const double* __restrict__ flux
                                                  double* __restrict__ rhs, long long tfp, long long npts,
                                                  const int* __restrict__ vM) {
     constexpr int N2 = N1 * N1, NP = N2 * N1;
-    for (long long v = blockIdx.x * (long long)kBlock + threadIdx.x; v < npts; v += (long long)gridDim.x * kBlock) {
+    for (long long v = xcd_block() * kBlock + threadIdx.x; v < npts; v += (long long)gridDim.x * kBlock) {
         const unsigned e = unsigned(v) / NP;  // volIdxMinus is 32-bit, so v is
         const int m = static_cast<int>(unsigned(v) - e * NP);
         const int i = m % N1, j = (m / N1) % N1, k = m / N2;
@@ -212,13 +217,13 @@ template <int N1>
 void launch_lifts(const double* flux, const double* dA, double* rhs, long long tfp, long long npts, const int* vM,
                   hipStream_t s) {
     if constexpr (N1 > 0)
-        hipLaunchKernelGGL(k_lift<N1>, dim3(grid_for(npts)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, vM);
+        hipLaunchKernelGGL(k_lift<N1>, dim3(grid_for_xcd(npts)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, vM);
     hipLaunchKernelGGL(k_lift_scatter<N1>, dim3(grid_for(tfp)), dim3(kBlock), 0, s, flux, dA, rhs, tfp, npts, vM);
 }
 
 __global__ void k_inv_mass(double* __restrict__ rhs, const double* __restrict__ jac, const double* __restrict__ w3,
                            int nxyz, long long npts, const double* __restrict__ eps, const double* __restrict__ mu) {
-    for (long long idx = blockIdx.x * (long long)blockDim.x + threadIdx.x; idx < npts; idx += (long long)gridDim.x * blockDim.x) {
+    for (long long idx = xcd_block() * blockDim.x + threadIdx.x; idx < npts; idx += (long long)gridDim.x * blockDim.x) {
         const long long e = npts <= 0x7fffffff ? unsigned(idx) / unsigned(nxyz) : idx / nxyz;
         const int i = static_cast<int>(idx - e * nxyz);
         const double ep = eps ? eps[e] : 1.0;
@@ -232,7 +237,7 @@ __global__ void k_inv_mass(double* __restrict__ rhs, const double* __restrict__ 
 __global__ void k_lsrk(double* __restrict__ st, double* __restrict__ k, const double* __restrict__ rhs, double a,
                        double b, double dt, long long npts, long long S) {
     const long long base = blockIdx.y * npts, sb = blockIdx.y * S;  // one component per grid row
-    for (long long p = blockIdx.x * (long long)blockDim.x + threadIdx.x; p < npts; p += (long long)gridDim.x * blockDim.x) {
+    for (long long p = xcd_block() * blockDim.x + threadIdx.x; p < npts; p += (long long)gridDim.x * blockDim.x) {
         const double ki = a * k[base + p] + dt * rhs[base + p];
         k[base + p] = ki;
         st[sb + p] += b * ki;
@@ -708,14 +713,14 @@ hipError_t launch_add_flux(const double* flux, const int* vM, const double* dA, 
 hipError_t launch_inv_mass(double* rhs, const double* jac, const double* w3, int nxyz, long long npts,
                            const double* eps, const double* mu, hipStream_t s) {
     if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_inv_mass, dim3(grid_for(npts)), dim3(kBlock), 0, s, rhs, jac, w3, nxyz, npts, eps, mu);
+    hipLaunchKernelGGL(k_inv_mass, dim3(grid_for_xcd(npts)), dim3(kBlock), 0, s, rhs, jac, w3, nxyz, npts, eps, mu);
     return hipGetLastError();
 }
 
 hipError_t launch_lsrk(double* st, double* k, const double* rhs, double a, double b, double dt,
                        long long npts, long long S, hipStream_t s) {
     if (npts <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_lsrk, dim3(grid_for(npts), 6), dim3(kBlock), 0, s, st, k, rhs, a, b, dt, npts, S);
+    hipLaunchKernelGGL(k_lsrk, dim3(grid_for_xcd(npts), 6), dim3(kBlock), 0, s, st, k, rhs, a, b, dt, npts, S);
     return hipGetLastError();
 }
 
