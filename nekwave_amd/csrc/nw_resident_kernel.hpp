@@ -156,7 +156,11 @@ void k_resident(ResidentArgs A) {
         wpq[t] = R(c_gll.w[N1][p] * c_gll.w[N1][q]);
     }
     __syncthreads();
-    if (sStop) return;  // uniform over the workgroup
+    // uniform over the workgroup: the second barrier, so that a wave that gives up later
+    // stores sStop only after every wave has read the entry value
+    const bool gone = sStop != 0;
+    __syncthreads();
+    if (gone) return;
 
     // Traces travel as 8-byte packets of 4 bytes of value and the epoch, stored and
     // read whole: a reader that sees the tag has the value, in one trip of the
