@@ -1079,7 +1079,47 @@ int Solver::step(double dt, int nsteps) {
     return st ? st : fin;
 }
 
+// Where a resident launch gave up, the events after it bracket launches that left at
+// once, and its steps ran again after the last event: the state is right, the times
+// are not.  They are taken again on the stage launches the solver keeps to from then
+// on, from a copy of the state (and of the probe records) that is put back afterwards.
 int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
+    const bool staged = staged_only;
+    int st = time_once(dt, warmup, nsteps, repeats, ms);
+    if (st || staged || !staged_only) return st;
+    const size_t ub = (prec == kFP64 ? 8 : 4) * 6 * size_t(stride);
+    struct {
+        void* live;
+        size_t bytes;
+        void* copy;
+    } kept[4] = {{d_u[0], ub, nullptr},
+                 {d_u[1], ub, nullptr},
+                 {nprobes > 0 ? d_probe_hist : nullptr, sizeof(double) * 6 * size_t(nprobes) * size_t(probe_cap), nullptr},
+                 {nprobes > 0 ? d_probe_slot : nullptr, sizeof(int), nullptr}};
+    const int cur[2] = {sets[0].cur, sets[1].cur};
+    const long long taken = probe_taken;
+    hipError_t he = hipSuccess;
+    for (auto& k : kept) {
+        if (k.live && st == NW_OK && he == hipSuccess && (st = dalloc(&k.copy, k.bytes)) == NW_OK)
+            he = hipMemcpyAsync(k.copy, k.live, k.bytes, hipMemcpyDeviceToDevice, stream);
+    }
+    const bool whole = st == NW_OK && he == hipSuccess;
+    if (whole) st = time_once(dt, warmup, nsteps, repeats, ms);
+    for (auto& k : kept)
+        if (k.live && whole && he == hipSuccess) he = hipMemcpyAsync(k.live, k.copy, k.bytes, hipMemcpyDeviceToDevice, stream);
+    if (he == hipSuccess) he = hipStreamSynchronize(stream);
+    sets[0].cur = cur[0];
+    sets[1].cur = cur[1];
+    probe_taken = taken;
+    for (auto& k : kept) {
+        if (k.copy) device_bytes -= (long long)k.bytes;
+        dfree(k.copy);
+    }
+    NW_TRY_HIP(he);
+    return st;
+}
+
+int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms) {
     if (!initialized || !uploaded) { set_error("time before create/upload"); return NW_ERR_STATE; }
     NW_CHECK_ARG(warmup >= 0 && nsteps >= 0 && repeats >= 1 && repeats <= 1024, "bad warmup/steps/repeats");
     NW_TRY_HIP(hipSetDevice(device));

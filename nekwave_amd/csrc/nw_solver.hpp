@@ -157,6 +157,7 @@ struct Solver {
     template <typename T>
     int upload_vec(T** dst, const std::vector<T>& v);
     int init_plain(const Mesh& m);
+    int time_once(double dt, int warmup, int nsteps, int repeats, double* ms);
     int set_dt(double dt);
     int set_of(int segment) const { return seg[size_t(segment)].parts.empty() ? 0 : 1; }
     int parity_of(const Instance& I) const { return sets[set_of(I.seg)].cur; }
