@@ -23,6 +23,8 @@
 #include <thread>
 #include <vector>
 
+#include <xmmintrin.h>
+
 #include "nw_plain.hpp"
 
 namespace nw {
@@ -120,12 +122,24 @@ hipError_t wait_event(hipEvent_t ev) {
     }
 }
 
+// The conversion below reads FP32 subnormals, which a thread whose MXCSR has
+// denormals-are-zero set (an option of some numerical libraries, inherited by the threads
+// it starts) would read as zeros.
+struct DefaultMxcsr {
+    const unsigned was = _mm_getcsr();
+    DefaultMxcsr() { _mm_setcsr(0x1f80); }
+    ~DefaultMxcsr() { _mm_setcsr(was); }
+};
+
 // Component block of n values from the slot (R) to the caller's array (FP64).
 template <typename R>
 void block_from_slot(double* host, const R* slot, size_t n) {
-    if constexpr (sizeof(R) == 8) std::memcpy(host, slot, n * 8);
-    else
+    if constexpr (sizeof(R) == 8) {
+        std::memcpy(host, slot, n * 8);
+    } else {
+        const DefaultMxcsr mode;
         for (size_t x = 0; x < n; ++x) host[x] = static_cast<double>(slot[x]);
+    }
 }
 
 // A state in chunks of nodes, taken by up to kStageSlots workers, each through its own
