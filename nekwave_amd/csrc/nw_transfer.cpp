@@ -278,9 +278,9 @@ int download_state(int device, hipStream_t s, double* host, long long P, const D
 int download_bytes(int device, hipStream_t s, void* host, const void* dev, size_t bytes) {
     Stage& st = stage();
     std::lock_guard<std::mutex> lk(st.mu);
-    const bool staged = bytes <= kStageBytes && ready_slot(st, device, 0) == hipSuccess;
+    const bool staged = bytes <= kStageBytes && !device_pointer(host) && ready_slot(st, device, 0) == hipSuccess;
     if (!staged) (void)hipGetLastError();
-    NW_TRY_HIP(hipMemcpyAsync(staged ? st.slot[0] : host, dev, bytes, hipMemcpyDeviceToHost, s));
+    NW_TRY_HIP(hipMemcpyAsync(staged ? st.slot[0] : host, dev, bytes, hipMemcpyDefault, s));
     NW_TRY_HIP(hipStreamSynchronize(s));
     if (staged) std::memcpy(host, st.slot[0], bytes);
     return NW_OK;

@@ -28,7 +28,8 @@ void stage_release();
 // order) or written.
 int upload_state(int device, hipStream_t s, const double* host, long long P, const DeviceState& d);
 int download_state(int device, hipStream_t s, double* host, long long P, const DeviceState& d);
-// `bytes` (any number) from device memory to host memory, in stream order, waited for.
+// `bytes` (any number) from device memory to the caller's array (host or device memory),
+// in stream order, waited for.
 int download_bytes(int device, hipStream_t s, void* host, const void* dev, size_t bytes);
 
 // Whether p is memory of a device (then the plain copies are used).
