@@ -219,6 +219,11 @@ int nw_mesh_locate_probes(const nw_mesh* m, int n, const double* xyz, int* elem,
  * precision, element count, single mesh or batch, whether the working set
  * exceeds the Infinity Cache, and groups_per_cu. */
 int nw_dg_tune(nw_dg* s);
+/* Extension: resident launches (meshes that fit on chip, any number of steps per launch)
+ * of this solver so far: those that completed, and those that gave up waiting for a
+ * place on the GPU, whose steps ran again by stage launches.  Both 0 where every step
+ * ran by stage launches.  Either output pointer may be NULL. */
+int nw_dg_resident_launches(const nw_dg* s, int64_t* completed, int64_t* gave_up);
 /* n1, element count and chosen elements per workgroup of segment `seg`. */
 int nw_dg_segment_info(const nw_dg* s, int seg, int* n1, int* nelt, int* epw);
 /* Extension: the tile option segment `seg` runs (0/1/2, as tuned or set),

@@ -198,6 +198,10 @@ class DgSolver {
     void setSegmentOption(int seg, int option, int streamK = -1) {
         check(nw_dg_set_segment_option(s_, seg, option, streamK));
     }
+    // Extension: resident launches that completed, and that gave up (nw_dg_resident_launches).
+    void residentLaunches(std::int64_t* completed, std::int64_t* gaveUp = nullptr) const {
+        check(nw_dg_resident_launches(s_, completed, gaveUp));
+    }
     // Extension: walk direction of the fused stages (nw_dg_set_walk / nw_dg_walk).
     void setWalk(int mode) { check(nw_dg_set_walk(s_, mode)); }
     bool alternatingWalk() const {

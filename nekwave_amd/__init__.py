@@ -356,6 +356,13 @@ class DgSolver:
         Cache) and keep the fastest (nw_dg_tune)."""
         check(lib().nw_dg_tune(self._handle()))
 
+    def residentLaunches(self):
+        """Resident launches of this solver so far: (completed, gave up)
+        (nw_dg_resident_launches); (0, 0) where every step ran by stage launches."""
+        done, lost = C.c_int64(), C.c_int64()
+        check(lib().nw_dg_resident_launches(self._handle(), C.byref(done), C.byref(lost)))
+        return done.value, lost.value
+
     def setSegmentOption(self, seg, option, stream_k=-1):
         """Set segment `seg`'s tile option and non-temporal k accesses (1, 0, or
         -1 for the default rule), e.g. as an earlier process tuned them

@@ -90,6 +90,7 @@ SIGNATURES = {
     "nw_dg_download_instance": (i, [vp, i, dp, sz]),
     "nw_dg_diag_instance": (i, [vp, i, C.POINTER(Diag)]),
     "nw_dg_tune": (i, [vp]),
+    "nw_dg_resident_launches": (i, [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "nw_dg_segment_info": (i, [vp, i, ip, ip, ip]),
     "nw_dg_segment_option": (i, [vp, i, ip, ip, ip]),
     "nw_dg_set_segment_option": (i, [vp, i, i, i]),

@@ -324,6 +324,12 @@ NW_API int nw_dg_walk(const nw_dg* s, int* alternating) {
     *alternating = s->s.alternating_walk() ? 1 : 0;
     return NW_OK;
 }
+NW_API int nw_dg_resident_launches(const nw_dg* s, int64_t* completed, int64_t* gave_up) {
+    NW_CHECK_ARG(s, "null solver");
+    if (completed) *completed = s->s.resident_done;
+    if (gave_up) *gave_up = s->s.resident_gave_up;
+    return NW_OK;
+}
 NW_API int nw_dg_segment_info(const nw_dg* s, int seg, int* n1, int* nelt, int* epw) {
     NW_CHECK_ARG(s && seg >= 0 && seg < (int)s->s.seg.size(), "bad segment");
     const nw::Segment& g = s->s.seg[seg];

@@ -1279,7 +1279,7 @@ int Solver::enqueue_resident(double dt, int nsteps) {
                 a.epoch = resident_epoch;
                 a.stop = d_stop;
                 a.stop_host = h_stop;
-                a.seq = ++resident_seq;
+                a.seq = resident_seq + 1;
                 a.spin_limit = env ? std::atoi(env) : 1 << 20;
                 a.dt = dt;
                 for (int s = 0; s < kStages; ++s) {
@@ -1288,6 +1288,7 @@ int Solver::enqueue_resident(double dt, int nsteps) {
                 }
                 resident_epoch += 5u * static_cast<unsigned>(n);
                 NW_TRY_HIP(launch_resident(sg.n1, prec, P.em, sg.affine, a, stream));
+                ++resident_seq;
             }
         }
         S.cur ^= 1;  // a launch reads one buffer and writes the other, whatever its steps
@@ -1313,8 +1314,10 @@ int Solver::finish() {
     if (!initialized) return NW_OK;
     hipError_t he = hipStreamSynchronize(stream);
     int st = NW_OK;
-    if (he == hipSuccess && !resident_log.empty() && *static_cast<volatile int*>(h_stop) != 0) {
-        const int seq = *static_cast<volatile int*>(h_stop);
+    const int seq = resident_log.empty() ? 0 : *static_cast<volatile int*>(h_stop);
+    if (he == hipSuccess) resident_done += seq != 0 ? seq - 1 : resident_seq;
+    if (he == hipSuccess && seq != 0) {
+        ++resident_gave_up;
         size_t c = resident_log.size() - 1;
         while (c > 0 && resident_log[c].seq > seq) --c;
         int left = 0;

@@ -98,6 +98,7 @@ struct Solver {
     bool staged_only = false;  // explicit launch shapes were asked for, or a resident launch gave up
     bool resident_held = false;  // this solver has the device's resident slot
     int resident_seq = 0;        // launches since the last finish()
+    long long resident_done = 0, resident_gave_up = 0;  // launches that completed, that gave up
     unsigned resident_epoch = 1;
     double resident_dt = 0.0;
     struct ResidentChunk {
