@@ -11,6 +11,8 @@
 namespace nw {
 namespace {
 
+constexpr int kLdsGranule = 1280;  // LDS is handed out in 128ths of a CU's 160 KB
+
 // LDS bytes of one workgroup, as k_resident declares them, without LSRK registers.
 constexpr int resident_lds(int n1, int em, int rsz, bool affine) {
     const int n2 = n1 * n1;
@@ -553,10 +555,12 @@ struct ResidentFamily {
         hipLaunchKernelGGL((k_resident<N1, EM, R, KR, AFF>), dim3(grid), dim3(N1 * N1 * N1), lds_k, s, a);
         return hipGetLastError();
     }
-    // Workgroups per CU that the hardware places wherever its waves start: the
-    // occupancy query counts wave slots, but a workgroup whose waves are no multiple
-    // of the four SIMDs loads them unevenly (six waves: 2 2 1 1), and two such may
-    // not fit where 12 slots are free.
+    // Workgroups per CU that the hardware places wherever its waves start.  The
+    // occupancy query divides the LDS by the bytes a workgroup asks for, but a workgroup
+    // is given whole granules (n1 = 4, eight elements: 15536 bytes take 16640, nine
+    // workgroups and not ten).  It counts wave slots, but a workgroup whose waves are no
+    // multiple of the four SIMDs loads them unevenly (six waves: 2 2 1 1), and two such
+    // may not fit where 12 slots are free.
     static int per_cu() {
         static std::atomic<int> known{-1};
         int n = known.load(std::memory_order_relaxed);
@@ -566,6 +570,8 @@ struct ResidentFamily {
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_resident<N1, EM, R, KR, AFF>, N1 * N1 * N1, lds_k) != hipSuccess ||
             hipFuncGetAttributes(&fa, fn) != hipSuccess)
             return 0;
+        const int lds = (static_cast<int>(fa.sharedSizeBytes) + lds_k + kLdsGranule - 1) / kLdsGranule * kLdsGranule;
+        n = std::min(n, 160 * 1024 / std::max(lds, kLdsGranule));
         constexpr int W = (N1 * N1 * N1 + 63) / 64;
         const int slots = 512 / ((std::max(fa.numRegs, 1) + 7) / 8 * 8);  // waves per SIMD
         if (W > 4 && W % 4 != 0) n = std::min(n, std::max(1, slots / ((W + 3) / 4)));

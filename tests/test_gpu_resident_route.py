@@ -27,10 +27,12 @@ def _box(n1, nel, jitter=0.1):
 @pytest.mark.parametrize("n1", range(2, 10))
 def test_resident_launches_complete_up_to_the_largest_mesh(n1, precision):
     for jitter in (0.0, 0.1):
-        for k in (1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 40, 48, 64, 80, 96, 128):  # multiples of 256 workgroups
+        for k in (1, 2, 3, 4, 6, 8, 12, 16, 20, 24, 32, 36, 40, 44, 48, 64, 72, 80, 88, 96, 128):  # multiples of 256 workgroups
             m = _box(n1, (16, 16, k), jitter)
             s = _solver(m, precision)
-            s.run(0.1 * m.computeMinNodeDistance(), 2)
+            # enough stages for every element to wait on every other: with a few, workgroups
+            # that were not placed at first would find room when others are through
+            s.run(0.1 * m.computeMinNodeDistance(), 40)
             done, lost = s.residentLaunches()
             s.finalize()
             assert lost == 0, (jitter, k)
