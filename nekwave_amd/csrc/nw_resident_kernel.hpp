@@ -29,7 +29,8 @@ template <int NT, int RBYTES>
 constexpr int resident_fit(int lds) {
     constexpr int waves = (NT + 63) / 64, eu = WavesPerEU<NT, RBYTES>::value;
     constexpr int regs = 4 * eu / waves > 1 ? 4 * eu / waves : 1;
-    return regs < 160 * 1024 / lds ? regs : 160 * 1024 / lds;
+    const int held = 160 * 1024 / ((lds + kLdsGranule - 1) / kLdsGranule * kLdsGranule);
+    return regs < held ? regs : held;
 }
 // Elements whose LSRK registers lie in LDS instead of VGPRs: enough that nothing spills (a
 // reload inside the stage waits for every packet in flight), as far as they fit beside
