@@ -14,14 +14,16 @@ ResidentKernel resident_kernel(int n1, int prec, int em, bool affine) {
 }
 }  // namespace
 
-long long resident_capacity(int n1, int prec, int em, bool affine, int max_per_cu) {
+ResidentCapacity resident_capacity(int n1, int prec, int em, bool affine, int max_per_cu) {
     const ResidentKernel k = resident_kernel(n1, prec, em, affine);
-    if (!k.per_cu) return 0;
+    if (!k.per_cu) return {};
     int dev = 0, cus = 0, per = k.per_cu();
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (hipGetDevice(&dev) != hipSuccess) return {};
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return {};
     if (max_per_cu > 0) per = std::min(per, max_per_cu);
-    return (long long)per * cus * resident_em(em);
+    const int most = resident_range(n1, prec, affine).per_cu;
+    const long long groups = (long long)per * cus, fits = groups * resident_em(em);
+    return {groups, most > 0 ? std::min(fits, (long long)most * cus) : fits};
 }
 
 hipError_t launch_resident(int n1, int prec, int em, bool affine, const ResidentArgs& a, hipStream_t s) {

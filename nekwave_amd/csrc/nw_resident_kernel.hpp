@@ -584,13 +584,15 @@ struct ResidentFamily {
 
 template <int N1, int EM, typename R, typename KR>
 ResidentKernel resident_pick(bool affine) {
-    if constexpr (resident_lds(N1, EM, sizeof(R), false) <= 160 * 1024) {
+    if constexpr (EM <= resident_range(N1, sizeof(R), sizeof(KR), true).em) {
         using A = ResidentFamily<N1, EM, R, KR, true>;
-        using G = ResidentFamily<N1, EM, R, KR, false>;
-        return affine ? ResidentKernel{&A::launch, &A::per_cu} : ResidentKernel{&G::launch, &G::per_cu};
-    } else {
-        return {};
+        if (affine) return {&A::launch, &A::per_cu};
     }
+    if constexpr (EM <= resident_range(N1, sizeof(R), sizeof(KR), false).em) {
+        using G = ResidentFamily<N1, EM, R, KR, false>;
+        if (!affine) return {&G::launch, &G::per_cu};
+    }
+    return {};
 }
 
 template <int N1, typename R, typename KR>

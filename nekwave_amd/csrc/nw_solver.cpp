@@ -1199,9 +1199,8 @@ void Solver::release_resident() {
 
 // The meshes of each segment that fit on chip, cut into launches of whole
 // meshes; the tables and buffers of those launches.  A segment takes resident
-// launches wherever all its meshes fit: measured faster at every size up to the
-// chip's (nw_resident_kernel.hpp), by least at the largest (n1 = 8, 1728 jittered
-// elements: 1.28x).  The smallest kernel size that holds a launch is taken (more
+// launches where all its meshes fit and they are the faster route (resident_range,
+// resident_fill).  The smallest kernel size that holds a launch is taken (more
 // workgroups per CU to overlap; n1 = 8, 1000 elements: two per workgroup 8.8 us per
 // stage, four 10.9).  Not with explicit launch shapes (tile option, segment choice,
 // walk), ghost faces or split BF16.  NW_RESIDENT=0: stage launches only (the two
@@ -1216,10 +1215,11 @@ int Solver::init_resident(const Mesh* const* meshes) {
     long long bytes = 0;
     for (size_t si = 0; si < seg.size(); ++si) {
         Segment& sg = seg[si];
-        long long cap[kResidentSizes], most = 0;
+        ResidentCapacity cap[kResidentSizes];
+        long long most = 0;
         for (int em = 0; em < kResidentSizes; ++em) {
             cap[em] = resident_capacity(sg.n1, prec, em, sg.affine, groups_per_cu);
-            most = std::max(most, cap[em]);
+            most = std::max(most, cap[em].elements);
         }
         std::vector<ResidentPart> parts;
         bool fits = true;
@@ -1232,12 +1232,17 @@ int Solver::init_resident(const Mesh* const* meshes) {
             parts.back().nelt += I.nelt;
         }
         if (!fits) continue;
+        long long places = 0, need = 0;
         for (ResidentPart& P : parts) {
-            while (cap[P.em] < P.nelt) ++P.em;
-            const long long groups = cap[P.em] / resident_em(P.em);
-            P.per = static_cast<int>((P.nelt + groups - 1) / groups);
-            bytes = std::max(bytes, resident_xchg_bytes(sg.n1, prec, P.nelt));
+            while (cap[P.em].elements < P.nelt) ++P.em;
+            P.per = static_cast<int>((P.nelt + cap[P.em].groups - 1) / cap[P.em].groups);
+            places += cap[P.em].groups * P.per;
+            need = std::max(need, resident_xchg_bytes(sg.n1, prec, P.nelt));
         }
+        if (parts.size() > 1 && (!resident_range(sg.n1, prec, sg.affine).several ||
+                                 double(sg.nelt) < resident_fill(sg.n1, sg.affine) * double(places)))
+            continue;
+        bytes = std::max(bytes, need);
         sg.parts = parts;
     }
     if (bytes == 0) return NW_OK;
