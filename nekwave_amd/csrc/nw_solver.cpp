@@ -919,18 +919,30 @@ std::map<TuneKey, std::pair<int, int>> g_tune;  // (tile option, non-temporal k)
 // read k) and keep the fastest.  The options alternate twice and each keeps its
 // best time, so a slow moment of the GPU does not decide.  Runs at a step
 // boundary, before graphs are captured.
-int Solver::tune() { return tune_segments(true); }
-
-// all: every segment; else those that only the staged launches run.
-int Solver::tune_segments(bool all) {
+int Solver::tune() {
     if (pipe != NW_PIPE_FUSED) return NW_OK;
     NW_TRY_HIP(hipSetDevice(device));
+    std::vector<int> segs(seg.size());
+    std::iota(segs.begin(), segs.end(), 0);
+    return tune_segments(segs);
+}
+
+// Before stage launches of a set: times its segments that were neither timed nor set.
+// (A segment that fits on chip comes here when its resident launches may not run.)
+int Solver::tune_untimed(const StageSet& S) {
+    std::vector<int> segs;
+    for (int x : S.segs)
+        if (autotune && !seg[size_t(x)].tuned) segs.push_back(x);
+    return segs.empty() ? NW_OK : tune_segments(segs);
+}
+
+int Solver::tune_segments(const std::vector<int>& segs) {
     // non-temporal k is a candidate only where the working set exceeds the
     // Infinity Cache (below it the hint only costs)
     const int nstream = fused_beyond_infinity_cache(working_set_bytes()) ? 2 : 1;
-    for (Segment& sg : seg) {
-        if (!all && !sg.parts.empty()) continue;
-        const int cur = sets[sg.parts.empty() ? 0 : 1].cur;
+    for (const int x : segs) {
+        Segment& sg = seg[size_t(x)];
+        const int cur = sets[set_of(x)].cur;
         const TuneKey key{device, sg.n1, prec, inst.size() == 1 ? 1 : 0, nstream - 1, groups_per_cu, sg.nelt};
         {
             std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -938,6 +950,7 @@ int Solver::tune_segments(bool all) {
             if (it != g_tune.end()) {
                 sg.option = it->second.first;
                 sg.stream = it->second.second;
+                sg.tuned = true;
                 continue;
             }
         }
@@ -993,11 +1006,11 @@ int Solver::tune_segments(bool all) {
                     sg.option = opt;
                     sg.stream = str;
                 }
+        sg.tuned = true;
         std::lock_guard<std::mutex> lk(g_tune_mu);
         g_tune[key] = {sg.option, sg.stream};
     }
     drop_graphs();  // captured launches carry the previous choices
-    tuned = true;
     return NW_OK;
 }
 
@@ -1010,7 +1023,7 @@ int Solver::set_segment_option(int s, int option, int stream_k) {
     NW_TRY_HIP(hipStreamSynchronize(stream));
     seg[size_t(s)].option = option;
     seg[size_t(s)].stream = stream_k;
-    tuned = true;  // an explicit choice stands until tune() is called
+    for (Segment& sg : seg) sg.tuned = true;  // an explicit choice stands until tune() is called
     staged_only = true;
     drop_graphs();
     return NW_OK;
@@ -1065,7 +1078,7 @@ int Solver::launch_steps(double dt, int nsteps) {
     if (nsteps == 0) return NW_OK;
     int st;
     const bool resident = hold_resident();
-    if (autotune && !tuned && !sets[0].segs.empty() && (st = tune_segments(false))) return st;
+    if ((st = tune_untimed(sets[0])) || (!resident && (st = tune_untimed(sets[1])))) return st;
     if (resident && (st = enqueue_resident(dt, nsteps))) return st;
     for (int x = 0; x < 2; ++x)
         if (!sets[x].segs.empty() && !(x == 1 && resident) && (st = enqueue_staged(sets[x], dt, nsteps))) return st;
@@ -1126,7 +1139,7 @@ int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms
     int st;
     // tune and capture outside the timed region
     const bool resident = hold_resident();
-    if (autotune && !tuned && !sets[0].segs.empty() && (st = tune_segments(false))) { finish(); return st; }
+    if ((st = tune_untimed(sets[0])) || (!resident && (st = tune_untimed(sets[1])))) { finish(); return st; }
     if (use_graph) {
         if ((st = set_dt(dt))) { finish(); return st; }
         for (int x = 0; x < 2; ++x)
@@ -1331,7 +1344,8 @@ int Solver::finish() {
         staged_only = true;
         *h_stop = 0;
         he = hipMemset(d_stop, 0, sizeof(int));
-        if (he == hipSuccess) st = enqueue_staged(sets[1], resident_dt, left);
+        if (he == hipSuccess) st = tune_untimed(sets[1]);
+        if (he == hipSuccess && st == NW_OK) st = enqueue_staged(sets[1], resident_dt, left);
         if (he == hipSuccess) he = hipStreamSynchronize(stream);
     }
     resident_log.clear();

@@ -30,6 +30,7 @@ struct Segment {
     int n1 = 0, nelt = 0, elem_base = 0, option = 0;
     int stream = -1;  // non-temporal k accesses: 1 / 0 as tuned, -1 the default rule (fused_stream_k)
     bool affine = false;  // every element a parallelepiped: records hold the geometry
+    bool tuned = false;   // option and stream were timed, or set by the caller
     long long node_base = 0;
     long long kbase = 0;                   // first k chunk (the most any tile option needs, after earlier segments)
     long long goff[kNumTileOptions] = {};  // offset of this segment's group order, per tile option
@@ -60,7 +61,7 @@ struct Solver {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int prec = 0, pipe = 1;
-    bool use_graph = true, initialized = false, uploaded = false, media = false, autotune = false, tuned = false;
+    bool use_graph = true, initialized = false, uploaded = false, media = false, autotune = false;
     int n1 = 0, np = 0, nelt = 0, kernels_per_step = 0;
     unsigned long long mesh_sig = 0;  // mesh_signature of a single-mesh solver's mesh
     long long npts = 0, tfp = 0, nhalo = 0, stride = 0, device_bytes = 0;
@@ -163,7 +164,8 @@ struct Solver {
     int set_of(int segment) const { return seg[size_t(segment)].parts.empty() ? 0 : 1; }
     int parity_of(const Instance& I) const { return sets[set_of(I.seg)].cur; }
     int init_resident(const Mesh* const* meshes);
-    int tune_segments(bool all);
+    int tune_segments(const std::vector<int>& segs);
+    int tune_untimed(const StageSet& S);
     int enqueue_staged(StageSet& S, double dt, int nsteps);
     int enqueue_resident(double dt, int nsteps);
     bool hold_resident();

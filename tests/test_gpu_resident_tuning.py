@@ -1,0 +1,42 @@
+"""Segments that fit on chip, where their resident launches may not run (here: a launch
+that gives up): they take the tuned shape of the stage launches like any other segment."""
+import numpy as np
+import pytest
+
+import nekwave_amd as nw
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, (9, 8, 7)), (4, (12, 11, 10)), (5, (10, 9, 8)), (6, (9, 8, 7))]
+
+
+def _solver(n1, nel):
+    m = nw.Mesh(n1)
+    m.createBoxMesh(*nel, 0, 1, 0, 1, 0, 1, True, False, False, jitter=0.1, seed=3)
+    s = nw.DgSolver(precision="fp32")
+    s.initialize(m, 1.0)
+    s.uploadState(np.random.default_rng(7).standard_normal(6 * m.getTotalPoints()))
+    return s
+
+
+def test_stage_launches_of_segments_that_fit_on_chip_are_tuned(monkeypatch):
+    picks, got = [], []
+    for shape in SHAPES:  # the choices, timed once per process
+        monkeypatch.setenv("NW_RESIDENT", "0")
+        s = _solver(*shape)
+        s.run(1e-4, 20)
+        picks.append(s.segments()[0]["option"])
+        want = s.downloadState()
+        s.finalize()
+        monkeypatch.delenv("NW_RESIDENT")
+        monkeypatch.setenv("NW_RESIDENT_SPINS", "0")
+        s = _solver(*shape)
+        assert s.segments()[0]["option"] == 0
+        s.run(1e-4, 20)
+        assert s.residentLaunches() == (0, 1)
+        got.append(s.segments()[0]["option"])
+        assert np.array_equal(s.downloadState(), want)
+        s.finalize()
+        monkeypatch.delenv("NW_RESIDENT_SPINS")
+    assert got == picks
+    assert any(picks), picks  # some order's pick is another shape than the first
