@@ -138,7 +138,8 @@ typedef struct nw_opts {
     int use_graph;    /* capture each step as a hipGraph (default 1) */
     int device;       /* HIP device ordinal (default 0) */
     int tile_option;  /* fused tile option 0/1/2 (elements per workgroup; at n1 = 8 in FP32,
-                       * 1 = matrix-core volume), -1 = tuned default */
+                       * 1 = matrix-core volume) by stage launches only; -1 (default) = tuned,
+                       * and resident launches where a mesh fits on chip */
     int groups_per_cu; /* extension, no counterpart in the reference: at most this many
                         * workgroups of a fused launch per CU (0 = as many as fit, the
                         * default), leaving room to other work on the device.  Results do
@@ -214,8 +215,9 @@ int nw_dg_probe_history(nw_dg* s, double* out, int max_records, int* nrecords);
 int nw_mesh_locate_probes(const nw_mesh* m, int n, const double* xyz, int* elem, double* rst);
 /* Autotuner: time every distinct tile option per segment -- with and without
  * non-temporal k accesses where the working set exceeds the 256 MiB Infinity
- * Cache -- and keep the fastest (runs by itself before the first step when
- * tile_option = -1).  Choices are kept per process, keyed by device, n1,
+ * Cache -- and keep the fastest (runs by itself before a segment's first stage launch
+ * when tile_option = -1).  It speaks of stage launches, as do the segment options and
+ * the walk below: whether a segment runs resident launches does not depend on them.  Choices are kept per process, keyed by device, n1,
  * precision, element count, single mesh or batch, whether the working set
  * exceeds the Infinity Cache, and groups_per_cu. */
 int nw_dg_tune(nw_dg* s);
@@ -226,21 +228,22 @@ int nw_dg_tune(nw_dg* s);
 int nw_dg_resident_launches(const nw_dg* s, int64_t* completed, int64_t* gave_up);
 /* n1, element count and chosen elements per workgroup of segment `seg`. */
 int nw_dg_segment_info(const nw_dg* s, int seg, int* n1, int* nelt, int* epw);
-/* Extension: the tile option segment `seg` runs (0/1/2, as tuned or set),
- * whether that option computes the volume contractions on the matrix cores
+/* Extension: the tile option of segment `seg`'s stage launches (0/1/2, as tuned or
+ * set; 0 before that: a segment that runs resident launches is timed by nw_dg_tune, or
+ * when its steps first run by stage launches), whether that option computes the volume contractions on the matrix cores
  * (n1 = 8 with FP32 fields, option 1; results equal the vector path's) and
  * whether its LSRK register accesses are non-temporal (tuned, or by default
  * where the working set exceeds the 256 MiB Infinity Cache and every wave
  * covers whole cache lines).  Any output pointer may be NULL. */
 int nw_dg_segment_option(const nw_dg* s, int seg, int* option, int* matrix_volume, int* stream_k);
-/* Extension: set segment `seg`'s tile option (0/1/2) and non-temporal k
- * accesses (1 on, 0 off, -1 the default rule) -- e.g. choices an earlier
+/* Extension: set the tile option (0/1/2) of segment `seg`'s stage launches and their
+ * non-temporal k accesses (1 on, 0 off, -1 the default rule) -- e.g. choices an earlier
  * process tuned and kept (nw_dg_segment_option).  The solver then counts as
  * tuned: autotuning does not override the choice until nw_dg_tune is called.
  * Results do not depend on either choice. */
 int nw_dg_set_segment_option(nw_dg* s, int seg, int option, int stream_k);
-/* Extension, no counterpart in the reference: the walk direction of the fused
- * stages.  mode 1: every other stage visits its element groups backwards, so it
+/* Extension, no counterpart in the reference: the walk direction of the stage
+ * launches.  mode 1: every other stage visits its element groups backwards, so it
  * starts on the groups the stage before it wrote last (some of them still in
  * the Infinity Cache; a batch then also takes its segments in reverse order);
  * 0: every stage forwards; -1 (default): alternate where the largest segment's

@@ -243,7 +243,8 @@ class DgSolver:
     """Reference DgSolver.  Extensions: precision ('fp64', 'fp32', 'fp32_k64'),
     pipeline ('fused', or 'plain' = FP64 from the reference's per-node and
     per-face-point arrays, any n1 in [2, 10]), graphs, the
-    fused tile option (-1: tuned) and groups_per_cu, a cap on the fused launch's
+    fused tile option (-1: tuned, and resident launches where the mesh fits on chip;
+    else stage launches of that option) and groups_per_cu, a cap on the fused launch's
     workgroups per CU (0: as many as fit)."""
 
     def __init__(self, precision="fp64", pipeline="fused", use_graph=True, device=0, tile_option=-1,
@@ -364,13 +365,13 @@ class DgSolver:
         return done.value, lost.value
 
     def setSegmentOption(self, seg, option, stream_k=-1):
-        """Set segment `seg`'s tile option and non-temporal k accesses (1, 0, or
-        -1 for the default rule), e.g. as an earlier process tuned them
+        """Set the tile option of segment `seg`'s stage launches and their
+        non-temporal k accesses (1, 0, or -1 for the default rule), e.g. as an earlier process tuned them
         (`segments()`); autotuning then keeps them until `tune()`."""
         check(lib().nw_dg_set_segment_option(self._handle(), int(seg), int(option), int(stream_k)))
 
     def setWalk(self, mode):
-        """Walk direction of the fused stages (nw_dg_set_walk): 1 every other
+        """Walk direction of the stage launches (nw_dg_set_walk): 1 every other
         stage backwards (a batch then also takes its segments in reverse
         order), 0 all forwards, -1 the default rule (alternate where the largest
         segment's working set exceeds the Infinity Cache by at most 8x)."""
@@ -383,9 +384,9 @@ class DgSolver:
         return bool(v.value)
 
     def segments(self):
-        """Per n1 segment: n1, elements, elements per workgroup, tile option,
-        whether it runs the volume contractions on the matrix cores and whether
-        its LSRK register accesses are non-temporal."""
+        """Per n1 segment: n1, elements, and of its stage launches elements per
+        workgroup, tile option, whether they run the volume contractions on the
+        matrix cores and whether their LSRK register accesses are non-temporal."""
         out = []
         for s in range(self.info()["segments"]):
             n1, nelt, epw = C.c_int(), C.c_int(), C.c_int()

@@ -1024,7 +1024,6 @@ int Solver::set_segment_option(int s, int option, int stream_k) {
     seg[size_t(s)].option = option;
     seg[size_t(s)].stream = stream_k;
     for (Segment& sg : seg) sg.tuned = true;  // an explicit choice stands until tune() is called
-    staged_only = true;
     drop_graphs();
     return NW_OK;
 }
@@ -1047,7 +1046,6 @@ int Solver::set_walk(int mode) {
     NW_TRY_HIP(hipSetDevice(device));
     NW_TRY_HIP(hipStreamSynchronize(stream));
     walk_mode = mode;
-    if (mode >= 0) staged_only = true;
     drop_graphs();  // captured launches carry the previous direction
     return NW_OK;
 }
@@ -1215,8 +1213,8 @@ void Solver::release_resident() {
 // launches where all its meshes fit and they are the faster route (resident_range,
 // resident_fill).  The smallest kernel size that holds a launch is taken (more
 // workgroups per CU to overlap; n1 = 8, 1000 elements: two per workgroup 8.8 us per
-// stage, four 10.9).  Not with explicit launch shapes (tile option, segment choice,
-// walk), ghost faces or split BF16.  NW_RESIDENT=0: stage launches only (the two
+// stage, four 10.9).  Not with a tile option, ghost faces or split BF16 (segment choices
+// and the walk speak of stage launches only).  NW_RESIDENT=0: stage launches only (the two
 // give the same bits; tests compare them).
 int Solver::init_resident(const Mesh* const* meshes) {
     const char* env = std::getenv("NW_RESIDENT");

@@ -96,7 +96,7 @@ struct Solver {
     int* d_gorder_rev = nullptr;  // the same walks with every sequence visited backwards
     int* d_ghead_rev = nullptr;
     // resident launches (sets[1])
-    bool staged_only = false;  // explicit launch shapes were asked for, or a resident launch gave up
+    bool staged_only = false;  // a resident launch gave up
     bool resident_held = false;  // this solver has the device's resident slot
     int resident_seq = 0;        // launches since the last finish()
     long long resident_done = 0, resident_gave_up = 0;  // launches that completed, that gave up

@@ -71,6 +71,28 @@ def test_where_stage_launches_are_faster(n1, precision, jitter, few, many):
             s.finalize()
 
 
+def test_choices_for_stage_launches_leave_resident_launches_on():
+    m = _box(5, (5, 4, 3))
+    a = _solver(m, "fp32")
+    a.run(1e-3, 2)
+    a.tune()
+    kept = a.segments()[0]
+    a.finalize()
+    # what a service applies in its next process
+    b = _solver(m, "fp32")
+    b.setSegmentOption(0, kept["option"], int(kept["stream_k"]))
+    seg = b.segments()[0]
+    assert (seg["option"], seg["stream_k"]) == (kept["option"], kept["stream_k"])
+    b.run(1e-3, 2)
+    b.setWalk(1)
+    b.run(1e-3, 2)
+    b.setWalk(-1)
+    b.tune()
+    b.run(1e-3, 2)
+    assert b.residentLaunches() == (3, 0)
+    b.finalize()
+
+
 def test_batches_of_several_launches():
     # (order, cavities of k^3, resident launches per run): one launch; several nearly full
     # ones; several half full; an order whose segments run staged beyond one launch
