@@ -219,7 +219,7 @@ void Solver::release() {
     allocs.clear();
     if (h_page) {
         (void)hipHostFree(h_page);
-        stage_release();
+        stage_release(device);
     }
     h_page = nullptr;
     h_stop = nullptr;
@@ -350,7 +350,7 @@ int Solver::init(const Mesh* const* meshes, int count, double c0_, const nw_opts
     if ((st = dalloc(reinterpret_cast<void**>(&d_dt), 8))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_diag_part), sizeof(double) * 3 * diag_blocks()))) return st;
     NW_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&h_page), 128, hipHostMallocDefault));
-    stage_retain();
+    stage_retain(device);
     h_stop = reinterpret_cast<int*>(h_page + 8);
     *h_stop = 0;
     long long max_inst = 0;

@@ -63,11 +63,24 @@ struct Job {
     }
 };
 
+// A pinned slot and the event of the kernel that last used it.
+struct Slot {
+    void* p = nullptr;
+    hipEvent_t ev = nullptr;
+};
+
+// Staging of one device.  A large transfer takes slot[] and the helpers for its whole
+// length, one at a time (two would share the link).  A small one (one worker) takes one
+// of small[] instead: it does not wait for another solver's large one (83 kB beside
+// downloads of 340 MB: 14 ms when it did).
 struct Stage {
-    std::mutex mu;  // held for a whole transfer
+    std::mutex mu;  // of slot[] and the job
+    Slot slot[kStageSlots];
+    std::mutex small_mu[kSmallSlots];
+    Slot small[kSmallSlots];
+    std::atomic<unsigned> turn{0};
+    std::mutex users_mu;
     int users = 0;
-    void* slot[kStageSlots] = {};
-    hipEvent_t ev[kMaxDevices][kStageSlots] = {};
     // helpers 1 .. kStageSlots - 1, started when a transfer first wants them
     std::vector<std::thread> helpers;
     std::mutex jm;
@@ -90,23 +103,40 @@ struct Stage {
             if (j && w < j->workers) j->run(w);
         }
     }
+    // A small slot that is free, or the next one in turn when it is.
+    std::unique_lock<std::mutex> take_small(int* which) {
+        for (int x = 0; x < kSmallSlots; ++x) {
+            std::unique_lock<std::mutex> lk(small_mu[x], std::try_to_lock);
+            if (lk.owns_lock()) {
+                *which = x;
+                return lk;
+            }
+        }
+        *which = static_cast<int>(turn.fetch_add(1) % kSmallSlots);
+        return std::unique_lock<std::mutex>(small_mu[*which]);
+    }
 };
-Stage& stage() {
-    static Stage* s = new Stage;  // never destroyed: no HIP calls after main
-    return *s;
+Stage& stage(int device) {
+    static Stage* s = new Stage[kMaxDevices];  // never destroyed: no HIP calls after main
+    return s[device];
 }
 
-// One slot and its event on the current device; with stage().mu held.
-hipError_t ready_slot(Stage& st, int device, int w) {
-    if (!st.slot[w]) {
-        const hipError_t e = hipHostMalloc(&st.slot[w], kStageBytes, hipHostMallocPortable);
+// A slot's memory and its event on the current device; with the slot's mutex held.
+hipError_t ready_slot(Slot& s) {
+    if (!s.p) {
+        const hipError_t e = hipHostMalloc(&s.p, kStageBytes, hipHostMallocPortable);
         if (e != hipSuccess) {
-            st.slot[w] = nullptr;
+            s.p = nullptr;
             return e;
         }
     }
-    if (!st.ev[device][w]) return hipEventCreateWithFlags(&st.ev[device][w], hipEventDisableTiming);
+    if (!s.ev) return hipEventCreateWithFlags(&s.ev, hipEventDisableTiming);
     return hipSuccess;
+}
+void free_slot(Slot& s) {
+    if (s.p) (void)hipHostFree(s.p);
+    if (s.ev) (void)hipEventDestroy(s.ev);
+    s = Slot();
 }
 
 // Waits for an event by asking for it: the runtime's own wait yields the CPU, and
@@ -147,8 +177,7 @@ void block_from_slot(double* host, const R* slot, size_t n) {
 template <typename R, bool UP>
 int move_state(int device, hipStream_t s, std::conditional_t<UP, const double*, double*> host, long long P,
                const DeviceState& d) {
-    Stage& st = stage();
-    std::lock_guard<std::mutex> lk(st.mu);
+    Stage& st = stage(device);
     const long long most = (long long)(kStageBytes / (6 * (UP ? 8 : sizeof(R))) / 64 * 64);
     // Helpers cost more where other threads want the CPUs, so no more than pay: on the
     // way out one worker per 6 MB of host array (FP32 leaves the link as twice that to
@@ -161,8 +190,11 @@ int move_state(int device, hipStream_t s, std::conditional_t<UP, const double*, 
     const long long per = P <= most && workers == 1 ? P : std::min(most, std::max<long long>(4096, P / (2 * workers) / 64 * 64));
     const long long chunks = (P + per - 1) / per;
     workers = static_cast<int>(std::min<long long>(workers, chunks));
+    int which = 0;
+    const std::unique_lock<std::mutex> lk = workers > 1 ? std::unique_lock<std::mutex>(st.mu) : st.take_small(&which);
+    Slot* const slots = workers > 1 ? st.slot : st.small + which;
     for (int w = 0; w < workers; ++w) {
-        const hipError_t e = ready_slot(st, device, w);
+        const hipError_t e = ready_slot(slots[w]);
         if (e != hipSuccess && w > 0) {  // fewer slots do
             (void)hipGetLastError();
             workers = w;
@@ -178,8 +210,8 @@ int move_state(int device, hipStream_t s, std::conditional_t<UP, const double*, 
     bool waits[kStageSlots] = {};  // a kernel that reads the worker's slot is in flight
     job->chunk = [&](int w, long long c) -> hipError_t {
         typedef std::conditional_t<UP, double, R> V;
-        V* slot = static_cast<V*>(st.slot[w]);
-        hipEvent_t ev = st.ev[device][w];
+        V* slot = static_cast<V*>(slots[w].p);
+        hipEvent_t ev = slots[w].ev;
         const long long p0 = c * per, n = std::min(per, P - p0);
         hipError_t e = hipSuccess;
         if constexpr (UP) {
@@ -198,7 +230,7 @@ int move_state(int device, hipStream_t s, std::conditional_t<UP, const double*, 
         }
         return e;
     };
-    job->end = [&](int w) -> hipError_t { return waits[w] ? wait_event(st.ev[device][w]) : hipSuccess; };
+    job->end = [&](int w) -> hipError_t { return waits[w] ? wait_event(slots[w].ev) : hipSuccess; };
     if (workers > 1) {
         std::lock_guard<std::mutex> jl(st.jm);
         try {
@@ -229,15 +261,15 @@ int move_state(int device, hipStream_t s, std::conditional_t<UP, const double*, 
 
 }  // namespace
 
-void stage_retain() {
-    Stage& st = stage();
-    std::lock_guard<std::mutex> lk(st.mu);
+void stage_retain(int device) {
+    Stage& st = stage(device);
+    std::lock_guard<std::mutex> lk(st.users_mu);
     ++st.users;
 }
 
-void stage_release() {
-    Stage& st = stage();
-    std::lock_guard<std::mutex> lk(st.mu);
+void stage_release(int device) {
+    Stage& st = stage(device);
+    std::lock_guard<std::mutex> lk(st.users_mu);  // no solver of the device is left to transfer
     if (--st.users > 0) return;
     {
         std::lock_guard<std::mutex> jl(st.jm);
@@ -247,15 +279,8 @@ void stage_release() {
     for (std::thread& t : st.helpers) t.join();
     st.helpers.clear();
     st.quit = false;
-    for (void*& p : st.slot) {
-        if (p) (void)hipHostFree(p);
-        p = nullptr;
-    }
-    for (auto& dev : st.ev)
-        for (hipEvent_t& e : dev) {
-            if (e) (void)hipEventDestroy(e);
-            e = nullptr;
-        }
+    for (Slot& s : st.slot) free_slot(s);
+    for (Slot& s : st.small) free_slot(s);
 }
 
 bool device_pointer(const void* p) {
@@ -276,13 +301,17 @@ int download_state(int device, hipStream_t s, double* host, long long P, const D
 }
 
 int download_bytes(int device, hipStream_t s, void* host, const void* dev, size_t bytes) {
-    Stage& st = stage();
-    std::lock_guard<std::mutex> lk(st.mu);
-    const bool staged = bytes <= kStageBytes && !device_pointer(host) && ready_slot(st, device, 0) == hipSuccess;
-    if (!staged) (void)hipGetLastError();
-    NW_TRY_HIP(hipMemcpyAsync(staged ? st.slot[0] : host, dev, bytes, hipMemcpyDefault, s));
+    int which = 0;
+    std::unique_lock<std::mutex> lk;
+    void* slot = nullptr;
+    if (bytes <= kStageBytes && !device_pointer(host)) {
+        lk = stage(device).take_small(&which);
+        if (ready_slot(stage(device).small[which]) == hipSuccess) slot = stage(device).small[which].p;
+        else (void)hipGetLastError();
+    }
+    NW_TRY_HIP(hipMemcpyAsync(slot ? slot : host, dev, bytes, hipMemcpyDefault, s));
     NW_TRY_HIP(hipStreamSynchronize(s));
-    if (staged) std::memcpy(host, st.slot[0], bytes);
+    if (slot) std::memcpy(host, slot, bytes);
     return NW_OK;
 }
 

@@ -14,14 +14,14 @@ struct DeviceState {
     long long cs, ns;
 };
 
-// Pinned staging of this process: up to kStageSlots slots of kStageBytes, made when
-// a transfer first needs them and freed when the last solver is gone.  One
-// transfer uses them at a time (transfers from several threads take turns: they
-// share the link anyway).
-constexpr int kStageSlots = 8;
+// Pinned staging, per device: up to kStageSlots slots of kStageBytes for a large transfer,
+// kSmallSlots for small ones, made when a transfer first needs them and freed when the
+// device's last solver is gone.  Large transfers of one device take turns (they share its
+// link); small ones and other devices' do not wait for them.
+constexpr int kStageSlots = 8, kSmallSlots = 4;
 constexpr size_t kStageBytes = size_t(2) << 20;
-void stage_retain();
-void stage_release();
+void stage_retain(int device);
+void stage_release(int device);
 
 // host (6 component blocks of P values, FP64) -> device, or back.  Returns when
 // the host array has been read (the device then holds the state in stream
