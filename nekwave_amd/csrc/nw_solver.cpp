@@ -3,8 +3,12 @@
 // for one mesh or a batch of independent meshes of mixed n1.
 #include "nw_solver.hpp"
 
+#include <fcntl.h>
+#include <sys/file.h>
+
 #include <algorithm>
 #include <atomic>
+#include <cerrno>
 #include <cmath>
 #include <cstdint>
 #include <cstdlib>
@@ -1190,21 +1194,51 @@ int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms
 // resident launches
 // ---------------------------------------------------------------------------
 namespace {
-// One resident launch at a time per device in this process: its workgroups wait
-// for each other, so two such grids that each hold part of the CUs would wait
-// until their polls run out.  Another solver's call meanwhile takes the staged
-// launches, which wait for nothing.
+// One resident launch at a time per device: its workgroups wait for each other, so two
+// such grids that each hold part of the CUs would wait until their polls run out.
+// Another solver's call meanwhile takes the stage launches, which wait for nothing.  In
+// this process a flag; between processes a lock on a file named after the device's PCI
+// address, which the system drops with a process that dies (0.4 us per call; where no
+// such file can be had, only this process's solvers are kept apart).
 std::atomic<bool> g_resident_busy[64];
+std::atomic<int> g_resident_file[64];  // descriptor + 1, 0: not opened yet, -1: none
+
+int resident_file(int device) {
+    int f = g_resident_file[device].load();
+    if (f == 0) {
+        char bus[32] = "";
+        int fd = -1;
+        if (hipDeviceGetPCIBusId(bus, sizeof bus, device) == hipSuccess) {
+            const std::string path = std::string("/tmp/nekwave_amd.") + bus + ".lock";
+            // opened for reading: enough for the lock, also where another user made it
+            fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);
+            if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CREAT | O_EXCL | O_CLOEXEC | O_NOFOLLOW, 0444);
+            if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);  // another process made it just now
+        } else {
+            (void)hipGetLastError();
+        }
+        f = fd >= 0 ? fd + 1 : -1;
+        g_resident_file[device].store(f);  // with the device's flag held: one thread at a time
+    }
+    return f - 1;
+}
 }  // namespace
 
 bool Solver::hold_resident() {
     if (staged_only || sets[1].segs.empty()) return false;
-    if (!resident_held) resident_held = !g_resident_busy[device].exchange(true, std::memory_order_acquire);
+    if (resident_held) return true;
+    if (g_resident_busy[device].exchange(true, std::memory_order_acquire)) return false;
+    const int fd = resident_file(device);
+    resident_held = fd < 0 || ::flock(fd, LOCK_EX | LOCK_NB) == 0 || errno != EWOULDBLOCK;
+    if (!resident_held) g_resident_busy[device].store(false, std::memory_order_release);
     return resident_held;
 }
 
 void Solver::release_resident() {
-    if (resident_held) g_resident_busy[device].store(false, std::memory_order_release);
+    if (!resident_held) return;
+    const int fd = resident_file(device);
+    if (fd >= 0) (void)::flock(fd, LOCK_UN);
+    g_resident_busy[device].store(false, std::memory_order_release);
     resident_held = false;
 }
 

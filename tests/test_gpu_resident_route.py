@@ -2,6 +2,9 @@
 faster route, and every one of them completes, from one workgroup per CU up to the largest
 mesh the launcher places (an overestimate would show as launches that give up, whose steps run again by stage
 launches with the same result), and one that gives up is counted as such."""
+import fcntl
+import glob
+
 import numpy as np
 import pytest
 
@@ -91,6 +94,29 @@ def test_choices_for_stage_launches_leave_resident_launches_on():
     b.run(1e-3, 2)
     assert b.residentLaunches() == (3, 0)
     b.finalize()
+
+
+def test_another_process_with_a_resident_launch():
+    m = _box(6, (6, 5, 4))
+    s = _solver(m, "fp32")
+    s.run(1e-4, 3)
+    # what another process holds during its resident calls on this device
+    held = [open(f) for f in glob.glob("/tmp/nekwave_amd.*.lock")]
+    assert held
+    for f in held:
+        fcntl.flock(f, fcntl.LOCK_EX | fcntl.LOCK_NB)  # free between calls
+    s.run(1e-4, 2)
+    assert s.residentLaunches() == (1, 0)
+    for f in held:
+        f.close()
+    s.run(1e-4, 2)
+    assert s.residentLaunches() == (2, 0)
+    got = s.downloadState()
+    s.finalize()
+    r = _solver(m, "fp32", tile_option=0)
+    r.run(1e-4, 7)
+    assert np.array_equal(got, r.downloadState())
+    r.finalize()
 
 
 def test_batches_of_several_launches():
