@@ -1300,9 +1300,17 @@ int Solver::init_resident(const Mesh* const* meshes) {
     return NW_OK;
 }
 
+// Polls before a workgroup of launch `n` (0: the first since the last wait) gives up.
+// NW_RESIDENT_SPINS, for tests: other bounds, per launch, the last one for all that follow.
+static int spin_limit(int n) {
+    const char* p = std::getenv("NW_RESIDENT_SPINS");
+    if (!p) return 1 << 20;
+    for (const char* c; n > 0 && (c = std::strchr(p, ',')); --n) p = c + 1;
+    return std::atoi(p);
+}
+
 int Solver::enqueue_resident(double dt, int nsteps) {
     const size_t rsz = prec == kFP64 ? 8 : 4;
-    const char* env = std::getenv("NW_RESIDENT_SPINS");  // a test's bound on the kernel's own waits
     StageSet& S = sets[1];
     resident_dt = dt;
     while (nsteps > 0) {
@@ -1330,7 +1338,7 @@ int Solver::enqueue_resident(double dt, int nsteps) {
                 a.stop = d_stop;
                 a.stop_host = h_stop;
                 a.seq = resident_seq + 1;
-                a.spin_limit = env ? std::atoi(env) : 1 << 20;
+                a.spin_limit = spin_limit(resident_seq);
                 a.dt = dt;
                 for (int s = 0; s < kStages; ++s) {
                     a.a[s] = kRkA[s];
