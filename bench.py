@@ -27,7 +27,8 @@ Profiling modes (short runs for rocprofv3): --profile-run (a few steps without
 graphs, then a 256 MiB copy as the byte-count calibration) and --profile-graph
 (one workload's graph timing alone, with the tile option and k policy given for a
 single mesh, tuned for the batch; --profile-workload picks the workload of either,
---profile-groups-per-cu caps the fused launches' workgroups per CU).
+--profile-groups-per-cu caps the fused launches' workgroups per CU); both profile the stage
+kernel, also where a mesh or a segment of the batch would run resident launches.
 """
 import argparse
 import json
@@ -93,7 +94,7 @@ def time_path(nw, wl, precision, pipeline, steps, warmup, repeats=5):
     t0 = time.perf_counter()
     ms = s.timeRepeats(wl.dt, steps, repeats, warmup=warmup)
     wall = time.perf_counter() - t0
-    info = s.info()
+    info = dict(s.info(), resident_launches=s.residentLaunches()[0])
     segs = s.segments() if hasattr(s, "segments") else None
     s.finalize()
     return [float(v) for v in ms], wall, info, segs
@@ -346,12 +347,17 @@ def other_config(nw, W, name, steps, error_steps=True):
         s_u, s_k = SIZES[prec]
         b = algorithmic_bytes_per_step(wl.npts, wl.nelt, s_u, s_k)
         out[prec] = {"dof_updates_per_s": 6 * wl.npts * steps / (ms * 1e-3), "ms_per_step": ms / steps,
-                     "ms_per_step_repeats": [r / steps for r in reps],
-                     "algorithmic_GBps": b / (ms / steps * 1e-3) / 1e9,
-                     "hbm_frac": b / (ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS,
-                     "kernels_per_step": info["kernels_per_step"]}
-        if segs:
-            out[prec]["segments"] = segs
+                     "ms_per_step_repeats": [r / steps for r in reps]}
+        if info["resident_launches"] > 0:
+            # segments on chip move their fields once per launch, not per stage: the bytes,
+            # launches and tile options of stage launches do not describe them
+            out[prec]["resident_launches"] = info["resident_launches"]
+        else:
+            out[prec].update({"algorithmic_GBps": b / (ms / steps * 1e-3) / 1e9,
+                              "hbm_frac": b / (ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS,
+                              "kernels_per_step": info["kernels_per_step"]})
+            if segs:
+                out[prec]["segments"] = segs
     if error_steps:
         n = wl.steps
         s64 = run_state(nw, wl, "fp64", n)
@@ -422,6 +428,8 @@ def main():
     import nekwave_amd as nw
     from nekwave_amd import workloads as W
 
+    if args.profile_graph or args.profile_run:
+        os.environ["NW_RESIDENT"] = "0"
     if args.profile_graph:
         profile_graph(nw, W, args.precision, args.steps, max(args.profile_option, 0), args.profile_stream,
                       workload=args.profile_workload, groups_per_cu=args.profile_groups_per_cu)
