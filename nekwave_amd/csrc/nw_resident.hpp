@@ -45,8 +45,8 @@ struct ResidentArgs {
 constexpr int kResidentSizes = 4;
 constexpr int resident_em(int em) { return 1 << em; }
 // Where resident launches beat the stage launches: the most elements per workgroup a
-// kernel is built for, (per_cu > 0) the most elements per CU it is used for, and whether a
-// segment of more meshes than fit at once takes several launches in turn.
+// kernel is built for, (per_cu > 0) the most elements per CU it is used for, and the most
+// launches in turn that a segment of more meshes than fit at once is cut into.
 //
 // Measured over whole ranges, boxes of 27 elements up to the chip's capacity (us per
 // stage, the stage kernel's tuned shape against this).  A kernel that spills registers
@@ -61,35 +61,45 @@ constexpr int resident_em(int em) { return 1 << em; }
 // 27.6) and a call of one step loses there (154 against 172 us: fields in and out of LDS).
 // Every other range won or drew (n1 = 4, FP32, 12288 jittered: 18.7 against 17.0; n1 = 8,
 // FP32, 2048: 22.4 against 15.2).
-// Against several launches stands one stage launch over the whole segment, which then
-// runs at its best rate: n1 = 5 lost throughout (124 elements per CU, FP32 affine 81.8
-// against 83.7, jittered 87.5 against 97.7, FP64 184 against 188 to 293), as did n1 = 4
-// with FP32 registers (78.9 against 85.5), n1 = 7 FP64 (202 against 211); the others won while
-// the launches were nearly full (n1 = 8 FP32 affine 1.16 to 1.23x, n1 = 9 1.08 to 1.16x).
+// Against several launches stands one stage launch over the whole segment, which runs at
+// its best rate from three or four times the chip's capacity on.  Batches of equal and of
+// mixed cavities, up to 40 launches: FP64 registers under FP32 fields won throughout
+// (affine 1.1 to 1.4x, jittered 1.06 to 1.3x) but at n1 = 5 and 7 jittered (0.69 to 1.2x);
+// affine FP64 won at n1 = 4, 6, 8, 9 (1.02 to 1.3x), affine FP32 from n1 = 6 on (1.0 to
+// 1.23x).  The rest lost or drew beyond a few launches (n1 = 5 FP64 0.70 to 0.97x, n1 = 7
+// jittered FP32 0.86 to 1.08x, at two launches 1.1 to 1.3x).
 struct ResidentRange {
-    int em, per_cu;
-    bool several;
+    int em, per_cu, launches;
 };
 constexpr ResidentRange resident_range(int n1, int rbytes, int kbytes, bool affine) {
-    const bool f64 = rbytes == 8, k32 = kbytes == 4;
+    const bool f64 = rbytes == 8, k32 = kbytes == 4, mixed = !f64 && !k32;
+    const int any = 1 << 30;
     switch (n1) {
-        case 2: return {f64 ? 0 : 1, 10, false};
-        case 3: return {1, f64 ? 5 : 8, false};
-        case 4: return {k32 ? (affine ? 8 : 4) : (affine ? 4 : 2), k32 && affine ? 60 : 0, !k32 && (affine || !f64)};
-        case 5: return {k32 && affine ? 8 : (k32 || affine ? 4 : 2), k32 && affine ? 28 : 0, false};
-        case 6: return {k32 ? 8 : 4, 0, true};
-        case 7: return {f64 && affine ? 8 : 4, 0, !f64};
-        case 8: return {!f64 && !k32 && !affine ? 2 : 4, 0, true};
-        default: return {f64 ? 2 : (k32 ? 8 : 4), 0, true};
+        case 2: return {f64 ? 0 : 1, 10, 1};
+        case 3: return {1, f64 ? 5 : 8, 1};
+        case 4: return {k32 ? (affine ? 8 : 4) : (affine ? 4 : 2), k32 && affine ? 60 : 0, mixed || (f64 && affine) ? any : k32 ? 2 : 1};
+        case 5: return {k32 && affine ? 8 : (k32 || affine ? 4 : 2), k32 && affine ? 28 : 0, mixed && affine ? any : 1};
+        case 6: return {k32 ? 8 : 4, 0, affine || mixed ? any : 3};
+        case 7: return {f64 && affine ? 8 : 4, 0, affine && !f64 ? any : 3};
+        case 8: return {mixed && !affine ? 2 : 4, 0, affine || !k32 ? any : 3};
+        default: return {f64 ? 2 : (k32 ? 8 : 4), 0, affine || mixed ? any : 3};
     }
 }
 constexpr ResidentRange resident_range(int n1, int prec, bool affine) {
     return resident_range(n1, prec == kFP64 ? 8 : 4, prec == kFP32 ? 4 : 8, affine);
 }
-// Several launches in turn: the share of their places that elements fill, at least (n1 =
-// 8, FP32, launches of 1331 elements where 1536 have places: affine 64.9 against 65.6,
-// jittered 65.1 against 70.0; n1 = 6, FP64 registers, affine, 1728 of 2048: 94.7 against 102.5).
-constexpr double resident_fill(int n1, bool affine) { return affine && n1 != 6 ? 0.8 : 0.9; }
+// Several launches in turn, n1 > 3: any number where the batch has segments of other orders
+// too and is larger than the Infinity Cache (`cold`), affine in FP32: a stage launch then
+// reads its segment from HBM (256 cavities of n1 = 4 to 9: the n1 = 4 and 5 segments
+// 34.5 and 75.6 us per stage against 29 and 66).
+constexpr int resident_launches(int n1, int prec, bool affine, bool cold) {
+    return cold && affine && prec == kFP32 && n1 > 3 ? 1 << 30 : resident_range(n1, prec, affine).launches;
+}
+// And the share of their places that elements fill, at least (n1 = 8, FP32, launches of
+// 1331 elements where 1536 have places: affine 64.9 against 65.6, jittered 65.1 against
+// 70.0; FP64 registers, affine, n1 = 6, 1728 of 2048: 94.7 against 102.5, n1 = 5, 3456 of
+// 3840: 102.7 against 114.5).
+constexpr double resident_fill(int n1, bool affine) { return !affine ? 0.9 : n1 == 5 || n1 == 6 ? 0.91 : 0.8; }
 
 // Workgroups of (n1, prec) with EM elements each on chip at once, at most `max_per_cu` per
 // CU (0: as many as fit), and the elements one launch takes.  0: not built (resident_range).

@@ -1257,6 +1257,7 @@ int Solver::init_resident(const Mesh* const* meshes) {
     std::vector<int> order(inst.size());
     std::iota(order.begin(), order.end(), 0);
     std::sort(order.begin(), order.end(), [&](int a, int b) { return inst[size_t(a)].elem_base < inst[size_t(b)].elem_base; });
+    const bool cold = seg.size() > 1 && fused_beyond_infinity_cache(working_set_bytes());
     long long bytes = 0;
     for (size_t si = 0; si < seg.size(); ++si) {
         Segment& sg = seg[si];
@@ -1284,7 +1285,7 @@ int Solver::init_resident(const Mesh* const* meshes) {
             places += cap[P.em].groups * P.per;
             need = std::max(need, resident_xchg_bytes(sg.n1, prec, P.nelt));
         }
-        if (parts.size() > 1 && (!resident_range(sg.n1, prec, sg.affine).several ||
+        if (parts.size() > 1 && ((long long)parts.size() > resident_launches(sg.n1, prec, sg.affine, cold) ||
                                  double(sg.nelt) < resident_fill(sg.n1, sg.affine) * double(places)))
             continue;
         bytes = std::max(bytes, need);

@@ -120,17 +120,29 @@ def test_another_process_with_a_resident_launch():
 
 
 def test_batches_of_several_launches():
-    # (order, cavities of k^3, resident launches per run): one launch; several nearly full
-    # ones; several half full; an order whose segments run staged beyond one launch
-    for n1, k, count, launches in ((8, 6, 8, 1), (8, 8, 12, 3), (7, 12, 2, 2), (5, 12, 6, 0), (5, 8, 8, 1)):
-        meshes = [_box(n1, (k, k, k), 0.0) for _ in range(count)]
-        b = nw.BatchSolver(precision="fp32")
+    # (order, jitter, precision, cavities of k^3, resident launches per run): one launch; several
+    # nearly full ones; too many for a jittered segment; places left empty; an order whose
+    # segments run staged beyond one launch
+    for n1, jitter, precision, k, count, launches in (
+            (8, 0.0, "fp32", 6, 8, 1), (8, 0.0, "fp32", 8, 12, 3), (8, 0.1, "fp32", 8, 12, 3), (8, 0.1, "fp32", 8, 16, 0),
+            (6, 0.0, "fp64", 11, 4, 0), (7, 0.0, "fp32", 12, 2, 2), (5, 0.0, "fp32", 12, 6, 0), (5, 0.0, "fp32", 8, 8, 1)):
+        meshes = [_box(n1, (k, k, k), jitter) for _ in range(count)]
+        b = nw.BatchSolver(precision=precision)
         b.initialize(meshes, 1.0)
         for x, m in enumerate(meshes):
             b.uploadState(x, np.ones(6 * m.getTotalPoints()))
         b.run(1e-3, 2)
-        assert b.residentLaunches() == (launches, 0), (n1, k)
+        assert b.residentLaunches() == (launches, 0), (n1, jitter, precision, k)
         b.finalize()
+    # the same order beside others, larger than the Infinity Cache together
+    meshes = [_box(5, (8, 8, 8), 0.0) for _ in range(56)] + [_box(6, (12, 12, 12), 0.0) for _ in range(9)]
+    b = nw.BatchSolver(precision="fp32")
+    b.initialize(meshes, 1.0)
+    for x, m in enumerate(meshes):
+        b.uploadState(x, np.ones(6 * m.getTotalPoints()))
+    b.run(1e-3, 1)
+    assert b.residentLaunches() == (4 + 3, 0)
+    b.finalize()
 
 
 def test_a_launch_that_gives_up_is_counted(monkeypatch):
