@@ -48,7 +48,7 @@ __device__ __forceinline__ long long xcd_block() { return (blockIdx.x & 7) * (gr
 // k_plain_stage, the t-lines in LDS like the others: a thread per column with its line
 // in registers had one or two waves per element and took 24.1 us at 593 thousand nodes,
 // n1 = 7, 22.6 at 373 thousand, n1 = 8, 21.0 at 512 thousand, n1 = 10; now 16.5, 11.9
-// and 15.2 (4.3 to 4.6 TB/s).
+// and 15.2 (4.3 to 4.6 TB/s; launch to launch, the kernel itself 13.5 at n1 = 7).
 template <int N1, int EPW, int KS>
 __global__ __launch_bounds__(EPW* KS* N1* N1) void k_volume_curl(const PlainVolumeArgs A) {
     constexpr int N2 = N1 * N1, NP = N1 * N2, T = KS * N2, NK = (N1 + KS - 1) / KS;

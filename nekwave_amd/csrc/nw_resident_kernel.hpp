@@ -40,7 +40,8 @@ constexpr int resident_fit(int lds) {
 // all in VGPRs -> this: FP32 jittered n1 = 5, 2744 elements 14.9 -> 10.9 us; FP64 jittered
 // n1 = 5, 1000 13.6 -> 9.6; FP32 with FP64 registers jittered n1 = 7, 1287 16.8 -> 15.1,
 // n1 = 5, 1728 10.2 -> 7.9.  Where nothing spills LDS costs 1-3 % (n1 = 9, 1000 elements
-// 16.2 -> 16.5), so the registers stay there.
+// 16.2 -> 16.5), so the registers stay there.  (tests/test_resident_registers.py reads the
+// spills from the built library, so that a compiler that spills more is noticed.)
 template <int N1, int EM, int RBYTES, int KBYTES, bool AFF>
 constexpr int resident_lds_k() {
     constexpr int NT = N1 * N1 * N1, fpt = (6 * N1 * N1 + NT - 1) / NT, kregs = 6 * KBYTES / 4;
@@ -73,12 +74,13 @@ __device__ __forceinline__ unsigned long long packet_load(const char* base, unsi
 // boundary's L2 write-back) and the chain of dependent first reads, not by
 // bandwidth.  Here the chain per stage is publish -> one trip of the fabric ->
 // flux -> two barriers.  Measured per stage, stage launches against this kernel:
-//   n1 = 5,   64 elements, FP64              6.7 ->  2.6 us
-//   n1 = 8,  216 / 512 elements, FP32        7.6 ->  2.7 / 10.5 -> 4.2 us
-//   n1 = 6, 1000 elements, FP64             14.5 ->  9.6 us
-//   n1 = 8, 1728 elements, FP32             21.6 -> 15.4 us (uniform), 23.7 -> 18.6 us (jittered)
-//   n1 = 9, 1728 elements, FP32, jittered   37.9 -> 29.0 us
-//   n1 = 4, 5832 elements, FP32             12.0 ->  8.2 us
+//   n1 = 5,   64 elements, FP64              6.5 ->  2.6 us
+//   n1 = 8,  216 / 512 elements, FP32        7.6 ->  2.5 / 10.3 -> 3.9 us
+//   n1 = 6, 1000 elements, FP64             14.2 ->  8.5 us
+//   n1 = 8, 1728 elements, FP32             21.7 -> 14.3 us (uniform), 23.3 -> 18.0 us (jittered)
+//   n1 = 9, 1728 elements, FP32             36.7 -> 27.4 us (uniform), 37.7 -> 29.6 us (jittered)
+//   n1 = 4, 5832 elements, FP32             11.8 ->  8.3 us
+// (where it is slower: resident_range).
 // Up to one element per workgroup the stage is bound by that chain (packets alone:
 // 1.3 us for 64 workgroups, 2.5 for 256, 4.3 for 512 at 384 points each); beyond, by
 // the vector ALUs (54-60 % busy) and LDS (55-60 %; n1 = 8 in FP32 77 % before QB).
@@ -96,8 +98,8 @@ void k_resident(ResidentArgs A) {
     // QB: contractions by quad broadcast (line8x3); wave k holds plane k.  Rows are 9
     // and planes 72 words apart there, so that lines in every direction and the nodes
     // of every face fall into different banks.  A third less
-    // LDS time (n1 = 8, 512 elements: 423 -> 285 LDS cycles per wave and stage), 4.6 ->
-    // 4.2 us per stage; 1728 uniform elements 17.0 -> 15.6.
+    // LDS time (n1 = 8, 512 elements: 423 -> 285 LDS cycles per wave and stage): against
+    // this kernel without it 4.6 -> 4.2 us per stage, 1728 uniform elements 17.0 -> 15.6.
     constexpr bool QB = N1 == 8 && sizeof(R) == 4;
     constexpr int RS = QB ? 9 : N1, PL = QB ? 72 : N2;  // row and plane strides of sU
     __shared__ R sU[EM][6][PL * N1];
