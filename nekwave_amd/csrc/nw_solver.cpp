@@ -7,7 +7,6 @@
 #include <sys/file.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cerrno>
 #include <cmath>
 #include <cstdint>
@@ -45,7 +44,12 @@ int upload_gll_tables(int device) {
 
 // LSRK45 coefficients, Carpenter & Kennedy (1994) (dg_solver.cpp:58-69).
 constexpr int kStages = 5;  // LSRK45 stages per step
-constexpr int kResidentSteps = 1024;        // steps of one resident launch, at most
+// Steps of one resident launch: about 10 ms of them, by 2.5 us per stage and 18 (FP32
+// fields) or 45 ns per thousand nodes.  Work of other streams waits for a launch's end, and
+// its fixed part (fields in and out, dispatch) is 10 to 60 us: 4 ms cost up to 1.2 %, 10 ms 0 to 0.7.
+// A call of many steps looks again whether the device is its own after kCallLaunches.
+constexpr double kLaunchUs = 10000.0, kStageUs = 2.5, kNodeUs32 = 18e-6, kNodeUs64 = 45e-6;
+constexpr int kCallLaunches = 3;
 // Uploads of this many values take the runtime's copy (38 GB/s pageable; 12.6 MB 0.38
 // against 0.45 ms staged); smaller ones the staging slots (one launch and one wait:
 // 0.4 MB 31 against 113 us), larger ones too (100 MB 2.2 against 3.7 ms).
@@ -227,7 +231,7 @@ void Solver::release() {
     }
     h_page = nullptr;
     h_stop = nullptr;
-    release_resident();
+    leave_call();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     ev0 = ev1 = nullptr;
@@ -1079,7 +1083,7 @@ int Solver::launch_steps(double dt, int nsteps) {
     NW_TRY_HIP(hipSetDevice(device));
     if (nsteps == 0) return NW_OK;
     int st;
-    const bool resident = hold_resident();
+    const bool resident = enter_call();
     if ((st = tune_untimed(sets[0])) || (!resident && (st = tune_untimed(sets[1])))) return st;
     if (resident && (st = enqueue_resident(dt, nsteps))) return st;
     for (int x = 0; x < 2; ++x)
@@ -1089,9 +1093,11 @@ int Solver::launch_steps(double dt, int nsteps) {
 }
 
 int Solver::step(double dt, int nsteps) {
-    const int st = launch_steps(dt, nsteps);
-    const int fin = finish();
-    return st ? st : fin;
+    for (;;) {
+        const int n = sets[1].segs.empty() ? nsteps : std::min(nsteps, kCallLaunches * resident_steps);
+        const int st = launch_steps(dt, n), fin = finish();
+        if (st || fin || (nsteps -= n) <= 0) return st ? st : fin;
+    }
 }
 
 // Where a resident launch gave up, the events after it bracket launches that left at
@@ -1140,7 +1146,7 @@ int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms
     NW_TRY_HIP(hipSetDevice(device));
     int st;
     // tune and capture outside the timed region
-    const bool resident = hold_resident();
+    const bool resident = enter_call();
     if ((st = tune_untimed(sets[0])) || (!resident && (st = tune_untimed(sets[1])))) { finish(); return st; }
     if (use_graph) {
         if ((st = set_dt(dt))) { finish(); return st; }
@@ -1194,52 +1200,77 @@ int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms
 // resident launches
 // ---------------------------------------------------------------------------
 namespace {
-// One resident launch at a time per device: its workgroups wait for each other, so two
-// such grids that each hold part of the CUs would wait until their polls run out.
-// Another solver's call meanwhile takes the stage launches, which wait for nothing.  In
-// this process a flag; between processes a lock on a file named after the device's PCI
-// address, which the system drops with a process that dies (0.4 us per call; where no
-// such file can be had, only this process's solvers are kept apart).
-std::atomic<bool> g_resident_busy[64];
-std::atomic<int> g_resident_file[64];  // descriptor + 1, 0: not opened yet, -1: none
+// Who steps on a device.  A resident launch has the GPU to itself: its workgroups wait for
+// each other, so two such grids that each hold part of the CUs would wait until their
+// polls run out, and another solver's stage launches would get one stage in between two
+// resident launches (measured: 100 steps of 512 elements 490 ms beside a solver of the
+// same size that kept to resident launches, 6 ms when both run stage launches).  So a call
+// runs resident only while no other solver's call is in progress on the device, and calls
+// that find another one share the device by stage launches.
+// Between processes by two files named after the device's PCI address, whose locks the
+// system drops with a process that dies: `turn`, held by a resident call, and `shared`,
+// held in common by calls with stage launches.  (0.7 us per call; where no such files can
+// be had, only this process's solvers are kept apart.)
+struct DeviceUse {
+    std::mutex mu;
+    int calls = 0, staged = 0;  // this process's calls in progress, and those by stage launches
+    bool opened = false;
+    int turn = -1, shared = -1;
+};
+DeviceUse g_use[64];
 
-int resident_file(int device) {
-    int f = g_resident_file[device].load();
-    if (f == 0) {
-        char bus[32] = "";
-        int fd = -1;
-        if (hipDeviceGetPCIBusId(bus, sizeof bus, device) == hipSuccess) {
-            const std::string path = std::string("/tmp/nekwave_amd.") + bus + ".lock";
-            // opened for reading: enough for the lock, also where another user made it
-            fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);
-            if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CREAT | O_EXCL | O_CLOEXEC | O_NOFOLLOW, 0444);
-            if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);  // another process made it just now
-        } else {
-            (void)hipGetLastError();
-        }
-        f = fd >= 0 ? fd + 1 : -1;
-        g_resident_file[device].store(f);  // with the device's flag held: one thread at a time
-    }
-    return f - 1;
+int lock_file(const char* bus, const char* what) {
+    const std::string path = std::string("/tmp/nekwave_amd.") + bus + "." + what + ".lock";
+    // opened for reading: enough for the lock, also where another user made it
+    int fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);
+    if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CREAT | O_EXCL | O_CLOEXEC | O_NOFOLLOW, 0444);
+    if (fd < 0) fd = ::open(path.c_str(), O_RDONLY | O_CLOEXEC | O_NOFOLLOW);  // another process made it just now
+    return fd;
+}
+bool try_lock(int fd) { return fd < 0 || ::flock(fd, LOCK_EX | LOCK_NB) == 0 || errno != EWOULDBLOCK; }
+void unlock(int fd) {
+    if (fd >= 0) (void)::flock(fd, LOCK_UN);
 }
 }  // namespace
 
-bool Solver::hold_resident() {
-    if (staged_only || sets[1].segs.empty()) return false;
-    if (resident_held) return true;
-    if (g_resident_busy[device].exchange(true, std::memory_order_acquire)) return false;
-    const int fd = resident_file(device);
-    resident_held = fd < 0 || ::flock(fd, LOCK_EX | LOCK_NB) == 0 || errno != EWOULDBLOCK;
-    if (!resident_held) g_resident_busy[device].store(false, std::memory_order_release);
+// At the start of a call that steps; true: by resident launches.
+bool Solver::enter_call() {
+    if (in_call) return resident_held;
+    DeviceUse& u = g_use[device];
+    std::lock_guard<std::mutex> lk(u.mu);
+    if (!u.opened) {
+        char bus[32] = "";
+        if (hipDeviceGetPCIBusId(bus, sizeof bus, device) == hipSuccess) {
+            u.turn = lock_file(bus, "resident");
+            u.shared = lock_file(bus, "staged");
+        } else {
+            (void)hipGetLastError();
+        }
+        u.opened = true;
+    }
+    in_call = true;
+    resident_held = u.calls++ == 0 && !staged_only && !sets[1].segs.empty() && try_lock(u.turn);
+    if (resident_held) {
+        if (try_lock(u.shared)) {
+            unlock(u.shared);
+        } else {  // another process's stage launches
+            unlock(u.turn);
+            resident_held = false;
+        }
+    }
+    // (not waited for: another process asks for it alone for a moment only)
+    if (!resident_held && u.staged++ == 0 && u.shared >= 0) (void)::flock(u.shared, LOCK_SH | LOCK_NB);
     return resident_held;
 }
 
-void Solver::release_resident() {
-    if (!resident_held) return;
-    const int fd = resident_file(device);
-    if (fd >= 0) (void)::flock(fd, LOCK_UN);
-    g_resident_busy[device].store(false, std::memory_order_release);
-    resident_held = false;
+void Solver::leave_call() {
+    if (!in_call) return;
+    DeviceUse& u = g_use[device];
+    std::lock_guard<std::mutex> lk(u.mu);
+    --u.calls;
+    if (resident_held) unlock(u.turn);
+    else if (--u.staged == 0) unlock(u.shared);
+    in_call = resident_held = false;
 }
 
 // The meshes of each segment that fit on chip, cut into launches of whole
@@ -1258,7 +1289,7 @@ int Solver::init_resident(const Mesh* const* meshes) {
     std::iota(order.begin(), order.end(), 0);
     std::sort(order.begin(), order.end(), [&](int a, int b) { return inst[size_t(a)].elem_base < inst[size_t(b)].elem_base; });
     const bool cold = seg.size() > 1 && fused_beyond_infinity_cache(working_set_bytes());
-    long long bytes = 0;
+    long long bytes = 0, most_nodes = 0;
     for (size_t si = 0; si < seg.size(); ++si) {
         Segment& sg = seg[si];
         ResidentCapacity cap[kResidentSizes];
@@ -1278,20 +1309,24 @@ int Solver::init_resident(const Mesh* const* meshes) {
             parts.back().nelt += I.nelt;
         }
         if (!fits) continue;
-        long long places = 0, need = 0;
+        long long places = 0, need = 0, nodes = 0;
         for (ResidentPart& P : parts) {
             while (cap[P.em].elements < P.nelt) ++P.em;
             P.per = static_cast<int>((P.nelt + cap[P.em].groups - 1) / cap[P.em].groups);
             places += cap[P.em].groups * P.per;
             need = std::max(need, resident_xchg_bytes(sg.n1, prec, P.nelt));
+            nodes = std::max(nodes, (long long)P.nelt * sg.n1 * sg.n1 * sg.n1);
         }
         if (parts.size() > 1 && ((long long)parts.size() > resident_launches(sg.n1, prec, sg.affine, cold) ||
                                  double(sg.nelt) < resident_fill(sg.n1, sg.affine) * double(places)))
             continue;
         bytes = std::max(bytes, need);
+        most_nodes = std::max(most_nodes, nodes);
         sg.parts = parts;
     }
     if (bytes == 0) return NW_OK;
+    const double stage_us = kStageUs + double(most_nodes) * (prec == kFP64 ? kNodeUs64 : kNodeUs32);
+    resident_steps = std::max(1, static_cast<int>(kLaunchUs / (kStages * stage_us)));
     int st;
     if ((st = upload_vec(&d_rnbr, nbr))) return st;
     if ((st = dalloc(reinterpret_cast<void**>(&d_xchg), size_t(bytes)))) return st;
@@ -1315,7 +1350,7 @@ int Solver::enqueue_resident(double dt, int nsteps) {
     StageSet& S = sets[1];
     resident_dt = dt;
     while (nsteps > 0) {
-        const int n = std::min(nsteps, nprobes > 0 ? std::min(kResidentSteps, snap_steps) : kResidentSteps);
+        const int n = std::min(nsteps, nprobes > 0 ? std::min(resident_steps, snap_steps) : resident_steps);
         resident_log.push_back({resident_seq + 1, S.cur, n});
         for (int x : S.segs) {
             const Segment& sg = seg[size_t(x)];
@@ -1391,7 +1426,7 @@ int Solver::finish() {
     }
     resident_log.clear();
     resident_seq = 0;
-    release_resident();
+    leave_call();
     if (he != hipSuccess) {
         set_error(std::string("hipStreamSynchronize: ") + hipGetErrorString(he));
         return NW_ERR_HIP;

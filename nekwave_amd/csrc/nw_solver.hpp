@@ -97,7 +97,8 @@ struct Solver {
     int* d_ghead_rev = nullptr;
     // resident launches (sets[1])
     bool staged_only = false;  // a resident launch gave up
-    bool resident_held = false;  // this solver has the device's resident slot
+    bool in_call = false, resident_held = false;  // between enter_call and leave_call; by resident launches
+    int resident_steps = 1;      // steps of one resident launch
     int resident_seq = 0;        // launches since the last finish()
     long long resident_done = 0, resident_gave_up = 0;  // launches that completed, that gave up
     unsigned resident_epoch = 1;
@@ -168,8 +169,8 @@ struct Solver {
     int tune_untimed(const StageSet& S);
     int enqueue_staged(StageSet& S, double dt, int nsteps);
     int enqueue_resident(double dt, int nsteps);
-    bool hold_resident();
-    void release_resident();
+    bool enter_call();
+    void leave_call();
     int launch_segment(const Segment& sg, int s, int parity, int option, int stream_k, hipStream_t st,
                        bool backwards = false);
     long long working_set_bytes() const;

@@ -31,8 +31,8 @@ def _solver(m, precision, **kw):
     return s
 
 
-# a launch takes 1024 steps at most: 2500 are three launches
-@pytest.mark.parametrize("spins,launches", [(None, (3, 0)), ("1000000,0", (1, 1)), ("1000000,1000000,0", (2, 1))])
+# a launch takes about 10 ms of steps, here 777, and a call waits after three of them
+@pytest.mark.parametrize("spins,launches", [(None, (4, 0)), ("1000000,0", (1, 1)), ("1000000,1000000,0", (2, 1))])
 def test_a_long_run_in_several_launches(spins, launches, monkeypatch):
     m = _box(3, (5, 4, 3))
     dt = 0.2 * m.computeMinNodeDistance()

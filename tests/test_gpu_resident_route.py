@@ -4,6 +4,8 @@ mesh the launcher places (an overestimate would show as launches that give up, w
 launches with the same result), and one that gives up is counted as such."""
 import fcntl
 import glob
+import threading
+import time
 
 import numpy as np
 import pytest
@@ -39,7 +41,7 @@ def test_resident_launches_complete_up_to_the_largest_mesh(n1, precision):
             done, lost = s.residentLaunches()
             s.finalize()
             assert lost == 0, (jitter, k)
-            assert done == 1 or (done == 0 and (k > 1 or (n1, precision) == (2, "fp64"))), (jitter, k)
+            assert done > 0 or k > 1 or (n1, precision) == (2, "fp64"), (jitter, k)
             if done == 0:  # does not fit, or stage launches are faster
                 break
 
@@ -96,15 +98,16 @@ def test_choices_for_stage_launches_leave_resident_launches_on():
     b.finalize()
 
 
-def test_another_process_with_a_resident_launch():
+# what another process holds during a call by resident launches, by stage launches
+@pytest.mark.parametrize("what,how", [("resident", fcntl.LOCK_EX), ("staged", fcntl.LOCK_SH)])
+def test_another_process_steps_on_the_device(what, how):
     m = _box(6, (6, 5, 4))
     s = _solver(m, "fp32")
     s.run(1e-4, 3)
-    # what another process holds during its resident calls on this device
-    held = [open(f) for f in glob.glob("/tmp/nekwave_amd.*.lock")]
+    held = [open(f) for f in glob.glob("/tmp/nekwave_amd.*.%s.lock" % what)]
     assert held
     for f in held:
-        fcntl.flock(f, fcntl.LOCK_EX | fcntl.LOCK_NB)  # free between calls
+        fcntl.flock(f, how | fcntl.LOCK_NB)  # free between calls
     s.run(1e-4, 2)
     assert s.residentLaunches() == (1, 0)
     for f in held:
@@ -117,6 +120,44 @@ def test_another_process_with_a_resident_launch():
     r.run(1e-4, 7)
     assert np.array_equal(got, r.downloadState())
     r.finalize()
+
+
+def test_solvers_of_one_device_share_it():
+    # a solver that could run resident launches all the time, beside one of a mesh that cannot
+    # (it gets a few stages in between two resident launches then: twenty times its time)
+    a, b = _solver(_box(5, (8, 8, 8)), "fp32"), _solver(_box(8, (20, 20, 20)), "fp32")
+    for s in (a, b):
+        s.tune()
+        s.run(1e-5, 20)
+
+    def timed(n):
+        t = []
+        for _ in range(n):
+            t0 = time.perf_counter()
+            b.run(1e-5, 20)
+            t.append(time.perf_counter() - t0)
+        return float(np.median(t))
+
+    alone = timed(9)
+    stop = threading.Event()
+
+    def keep_stepping():
+        while not stop.is_set():
+            a.run(1e-5, 100)
+
+    th = threading.Thread(target=keep_stepping)
+    th.start()
+    try:
+        time.sleep(0.05)
+        beside = timed(9)
+    finally:
+        stop.set()
+        th.join()
+    assert a.residentLaunches()[1] == 0
+    # an equal share of the GPU is twice the time alone, a launch in hand at the start some more
+    assert beside < 6 * alone, (beside, alone)
+    a.finalize()
+    b.finalize()
 
 
 def test_batches_of_several_launches():
