@@ -1092,9 +1092,16 @@ int Solver::launch_steps(double dt, int nsteps) {
     return NW_OK;
 }
 
+// The device is given back also where an exception leaves the call (finish() does it else).
+struct Solver::Call {
+    Solver* s;
+    ~Call() { s->leave_call(); }
+};
+
 int Solver::step(double dt, int nsteps) {
+    const Call call{this};
     for (;;) {
-        const int n = sets[1].segs.empty() ? nsteps : std::min(nsteps, kCallLaunches * resident_steps);
+        const int n = sets[1].segs.empty() || staged_only ? nsteps : std::min(nsteps, kCallLaunches * resident_steps);
         const int st = launch_steps(dt, n), fin = finish();
         if (st || fin || (nsteps -= n) <= 0) return st ? st : fin;
     }
@@ -1145,6 +1152,7 @@ int Solver::time_once(double dt, int warmup, int nsteps, int repeats, double* ms
     NW_CHECK_ARG(warmup >= 0 && nsteps >= 0 && repeats >= 1 && repeats <= 1024, "bad warmup/steps/repeats");
     NW_TRY_HIP(hipSetDevice(device));
     int st;
+    const Call call{this};
     // tune and capture outside the timed region
     const bool resident = enter_call();
     if ((st = tune_untimed(sets[0])) || (!resident && (st = tune_untimed(sets[1])))) { finish(); return st; }

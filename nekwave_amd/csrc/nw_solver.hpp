@@ -155,6 +155,7 @@ struct Solver {
     DeviceState state_of(const Instance& I) const;
 
    private:
+    struct Call;
     int dalloc(void** p, size_t bytes);
     void dfree(void* p);
     template <typename T>
