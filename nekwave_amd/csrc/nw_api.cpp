@@ -208,6 +208,7 @@ NW_API void nw_opts_default(nw_opts* o) {
 
 NW_API int nw_dg_create(const nw_mesh* m, double c0, const nw_opts* opts, nw_dg** out) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(m && out, "null argument");
     *out = nullptr;
     nw_opts o;
@@ -227,6 +228,7 @@ NW_API int nw_dg_create(const nw_mesh* m, double c0, const nw_opts* opts, nw_dg*
 
 NW_API int nw_batch_create(int count, const nw_mesh* const* meshes, double c0, const nw_opts* opts, nw_dg** out) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(meshes && out && count >= 1, "bad argument");
     *out = nullptr;
     nw_opts o;
@@ -250,44 +252,52 @@ NW_API int nw_batch_create(int count, const nw_mesh* const* meshes, double c0, c
 
 NW_API int nw_dg_upload(nw_dg* s, const double* host, size_t n) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.upload(0, host, n);
     NW_GUARD_END
 }
 NW_API int nw_dg_download(nw_dg* s, double* host, size_t n) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.download(0, host, n);
     NW_GUARD_END
 }
 NW_API int nw_dg_upload_instance(nw_dg* s, int instance, const double* host, size_t n) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.upload(instance, host, n);
     NW_GUARD_END
 }
 NW_API int nw_dg_download_instance(nw_dg* s, int instance, double* host, size_t n) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.download(instance, host, n);
     NW_GUARD_END
 }
 NW_API int nw_dg_rel_l2(nw_dg* s, int instance, const double* ref, size_t n, double* rel_l2) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.rel_l2(instance, ref, n, rel_l2);
 }
 NW_API int nw_dg_set_probes(nw_dg* s, const nw_mesh* m, int n, const double* xyz, int capacity) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s && m, "null argument");
     return s->s.set_probes(m->m, n, xyz, capacity);
     NW_GUARD_END
 }
 NW_API int nw_dg_probe_sample(nw_dg* s) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.probe_sample();
 }
 NW_API int nw_dg_probe_history(nw_dg* s, double* out, int max_records, int* nrecords) {
     NW_GUARD_BEGIN
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s, "null solver");
     return s->s.probe_history(out, max_records, nrecords);
     NW_GUARD_END
@@ -298,6 +308,7 @@ NW_API int nw_mesh_locate_probes(const nw_mesh* m, int n, const double* xyz, int
     return NW_OK;
 }
 NW_API int nw_dg_diag_instance(nw_dg* s, int instance, nw_diag* out) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s && out, "null argument");
     return s->s.diag(instance, out);
 }
@@ -379,6 +390,7 @@ NW_API int nw_dg_sync(nw_dg* s) {
     return NW_OK;
 }
 NW_API int nw_dg_diag(nw_dg* s, nw_diag* out) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(s && out, "null argument");
     return s->s.diag(0, out);
 }
@@ -398,7 +410,10 @@ NW_API int nw_dg_get_info(const nw_dg* s, nw_dg_info* o) {
     o->kernels_per_step = s->s.kernels_per_step;
     return NW_OK;
 }
-NW_API void nw_dg_destroy(nw_dg* s) { delete s; }
+NW_API void nw_dg_destroy(nw_dg* s) {
+    const nw::NoCapture nc;
+    delete s;
+}
 
 // -------------------------------------------------------- kernel level ----
 static hipStream_t hs(void* s) { return static_cast<hipStream_t>(s); }
@@ -493,6 +508,7 @@ NW_API int nw_launch_diagnostics(const double* st, int64_t S, const double* jac,
         std::lock_guard<std::mutex> lk(g_part_mu);
         if (!g_part[dev]) {
             void* p = nullptr;
+            const nw::NoCapture nc;
             if (hipMalloc(&p, sizeof(double) * 3 * nw::kEnergyMaxBlocks) != hipSuccess) {
                 set_error("diagnostics: hipMalloc of the partial sums failed");
                 return NW_ERR_ALLOC;
@@ -593,6 +609,7 @@ NW_API int nw_rand_normal(uint64_t seed, size_t n, double* out) {
 
 // ------------------------------------------------------------- device ----
 NW_API int nw_dev_alloc(size_t bytes, void** p) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(p, "null out");
     int st = ensure_tables();
     if (st) return st;
@@ -600,22 +617,27 @@ NW_API int nw_dev_alloc(size_t bytes, void** p) {
     return NW_OK;
 }
 NW_API int nw_dev_free(void* p) {
+    const nw::NoCapture nc;
     NW_TRY_HIP(hipFree(p));
     return NW_OK;
 }
 NW_API int nw_dev_h2d(void* dst, const void* src, size_t bytes) {
+    const nw::NoCapture nc;
     NW_TRY_HIP(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
     return NW_OK;
 }
 NW_API int nw_dev_d2h(void* dst, const void* src, size_t bytes) {
+    const nw::NoCapture nc;
     NW_TRY_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return NW_OK;
 }
 NW_API int nw_dev_sync(void) {
+    const nw::NoCapture nc;
     NW_TRY_HIP(hipDeviceSynchronize());
     return NW_OK;
 }
 NW_API int nw_bench_copy(size_t bytes, int reps, double* ms) {
+    const nw::NoCapture nc;
     NW_CHECK_ARG(ms && reps > 0 && bytes >= 16, "bad argument");
     void *a = nullptr, *b = nullptr;
     NW_TRY_HIP(hipMalloc(&a, bytes));

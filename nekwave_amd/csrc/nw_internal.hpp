@@ -65,4 +65,19 @@ inline int face_code_neighbor(int e, int f) { return e * 8 + f; }
 int upload_gll_tables(int device);
 const GllTables& host_gll_tables();
 
+// While one thread captures a stream, a synchronous copy or an allocation of another
+// thread fails and breaks the capture.  A solver's capture of its step holds Capture;
+// entry points that make such calls hold NoCapture, any number at once, none of them
+// while a capture is waiting or in progress.  Neither nests.
+struct NoCapture {
+    NoCapture();
+    ~NoCapture();
+    NoCapture(const NoCapture&) = delete;
+};
+struct Capture {
+    Capture();
+    ~Capture();
+    Capture(const Capture&) = delete;
+};
+
 }  // namespace nw

@@ -15,12 +15,32 @@
 #include <map>
 #include <mutex>
 #include <numeric>
+#include <shared_mutex>
 #include <vector>
 
 #include "nw_fused.hpp"
 #include "nw_plain.hpp"
 
 namespace nw {
+
+namespace {
+std::mutex g_capture_gate;  // held by a capture from its wait on
+std::shared_mutex g_capture;
+}  // namespace
+
+NoCapture::NoCapture() {
+    std::lock_guard<std::mutex> lk(g_capture_gate);
+    g_capture.lock_shared();
+}
+NoCapture::~NoCapture() { g_capture.unlock_shared(); }
+Capture::Capture() {
+    g_capture_gate.lock();
+    g_capture.lock();
+}
+Capture::~Capture() {
+    g_capture.unlock();
+    g_capture_gate.unlock();
+}
 
 namespace {
 std::mutex g_tables_mu;
@@ -606,8 +626,7 @@ DeviceState Solver::state_of(const Instance& I) const {
 
 int Solver::set_dt(double dt) {
     if (dt == last_dt) return NW_OK;
-    NW_TRY_HIP(hipStreamSynchronize(stream));
-    NW_TRY_HIP(hipMemcpy(d_dt, &dt, sizeof(double), hipMemcpyHostToDevice));
+    NW_TRY_HIP(launch_fill(d_dt, 1, dt, stream));  // in stream order
     last_dt = dt;
     return NW_OK;
 }
@@ -873,6 +892,7 @@ int Solver::probe_history(double* host, int max_records, int* nrecords) {
 }
 
 int Solver::build_graph(StageSet& S, int parity) {
+    const Capture alone;
     hipGraph_t g = nullptr;
     NW_TRY_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
     int st = enqueue_step(S, parity);
@@ -1128,6 +1148,7 @@ int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
     const long long taken = probe_taken;
     hipError_t he = hipSuccess;
     for (auto& k : kept) {
+        const NoCapture nc;
         if (k.live && st == NW_OK && he == hipSuccess && (st = dalloc(&k.copy, k.bytes)) == NW_OK)
             he = hipMemcpyAsync(k.copy, k.live, k.bytes, hipMemcpyDeviceToDevice, stream);
     }
@@ -1140,6 +1161,7 @@ int Solver::time(double dt, int warmup, int nsteps, int repeats, double* ms) {
     sets[1].cur = cur[1];
     probe_taken = taken;
     for (auto& k : kept) {
+        const NoCapture nc;
         if (k.copy) device_bytes -= (long long)k.bytes;
         dfree(k.copy);
     }
@@ -1427,7 +1449,7 @@ int Solver::finish() {
         sets[1].cur = resident_log[c].cur;
         staged_only = true;
         *h_stop = 0;
-        he = hipMemset(d_stop, 0, sizeof(int));
+        he = launch_zero_int(d_stop, stream);
         if (he == hipSuccess) st = tune_untimed(sets[1]);
         if (he == hipSuccess && st == NW_OK) st = enqueue_staged(sets[1], resident_dt, left);
         if (he == hipSuccess) he = hipStreamSynchronize(stream);
