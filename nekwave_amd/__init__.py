@@ -492,7 +492,8 @@ class FieldWriter:
 class BatchSolver(DgSolver):
     """Many independent meshes (any mix of n1, common dt) in one solver: each
     stage launches one persistent fused kernel per n1 segment, one after
-    another.  Instances are addressed by their index in the list given to
+    another, or a segment runs resident launches of the meshes that fit on chip at
+    once.  Instances are addressed by their index in the list given to
     initialize()."""
 
     def __init__(self, precision="fp32", use_graph=True, device=0, tile_option=-1, groups_per_cu=0):
